@@ -849,6 +849,110 @@ int les::finish(les_ctx* c) {
     return first == hipSuccess ? LES_OK : LES_E_HIP;
 }
 
+// ---- host transfers ------------------------------------------------------------
+// hipMemcpy2DAsync moves pageable memory a row at a time, about 7.4 us a row
+// whatever its length (128 x 128 x 66 levels: 62 ms for 8.6 MB each way).  A
+// block without row padding is one contiguous copy (0.3 - 0.5 ms there).  A
+// strided block in pageable memory (the reference's ldx = nxt + 2 arrays)
+// goes through two page-locked chunks: the rows of one are packed or
+// unpacked on the host while the other is in flight; the caller's padding
+// columns are neither read nor written.  A strided block in memory the
+// runtime knows (page-locked, managed) keeps the 2-D copy, which takes it
+// whole.
+namespace {
+constexpr size_t BOUNCE = (size_t)1 << 17;   // doubles per chunk (1 MiB)
+
+bool pageable(const void* h) {
+    hipPointerAttribute_t a;
+    std::memset(&a, 0, sizeof(a));
+    const hipError_t e = hipPointerGetAttributes(&a, h);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // memory the runtime does not know
+        return true;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+}
+
+// the chunks, free for use; false when a row does not fit or none can be had
+bool bounce_ready(les_ctx* c) {
+    if ((size_t)c->nx > BOUNCE) return false;
+    for (int i = 0; i < 2; ++i) {
+        if (!c->bounce[i]) {
+            void* p = nullptr;
+            if (hipHostMalloc(&p, sizeof(double) * BOUNCE, hipHostMallocDefault) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
+            c->bounce[i] = static_cast<double*>(p);
+        }
+        if (!c->ev_bounce[i] && hipEventCreateWithFlags(&c->ev_bounce[i], hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            c->ev_bounce[i] = nullptr;
+            return false;
+        }
+        les_note(c, hipEventSynchronize(c->ev_bounce[i]));
+    }
+    return true;
+}
+}  // namespace
+
+void les::rows_h2d(les_ctx* c, double* d, const double* h, int ld, long rows) {
+    const size_t nx = (size_t)c->nx;
+    if (rows <= 0) return;
+    if ((size_t)ld == nx) {
+        les_note(c, hipMemcpyAsync(d, h, nx * 8 * (size_t)rows, hipMemcpyHostToDevice, c->stream));
+        return;
+    }
+    if (!pageable(h) || !bounce_ready(c)) {
+        les_note(c, hipMemcpy2DAsync(d, nx * 8, h, (size_t)ld * 8, nx * 8, (size_t)rows, hipMemcpyHostToDevice,
+                                     c->stream));
+        return;
+    }
+    const long per = (long)(BOUNCE / nx);
+    int b = 0;
+    for (long r0 = 0; r0 < rows; r0 += per, b ^= 1) {
+        const long n = std::min(per, rows - r0);
+        les_note(c, hipEventSynchronize(c->ev_bounce[b]));
+        for (long r = 0; r < n; ++r)
+            std::memcpy(c->bounce[b] + (size_t)r * nx, h + (size_t)(r0 + r) * (size_t)ld, nx * 8);
+        les_note(c, hipMemcpyAsync(d + (size_t)r0 * nx, c->bounce[b], (size_t)n * nx * 8, hipMemcpyHostToDevice,
+                                   c->stream));
+        les_note(c, hipEventRecord(c->ev_bounce[b], c->stream));
+    }
+    // the caller may change its rows after the call; the chunks are waited
+    // for by the next transfer or finish()
+}
+
+void les::rows_d2h(les_ctx* c, double* h, const double* d, int ld, long rows) {
+    const size_t nx = (size_t)c->nx;
+    if (rows <= 0) return;
+    if ((size_t)ld == nx) {
+        les_note(c, hipMemcpyAsync(h, d, nx * 8 * (size_t)rows, hipMemcpyDeviceToHost, c->stream));
+        return;
+    }
+    if (!pageable(h) || !bounce_ready(c)) {
+        les_note(c, hipMemcpy2DAsync(h, (size_t)ld * 8, d, nx * 8, nx * 8, (size_t)rows, hipMemcpyDeviceToHost,
+                                     c->stream));
+        return;
+    }
+    const long per = (long)(BOUNCE / nx);
+    auto fetch = [&](long r0, int b) {
+        const long n = std::min(per, rows - r0);
+        les_note(c, hipMemcpyAsync(c->bounce[b], d + (size_t)r0 * nx, (size_t)n * nx * 8, hipMemcpyDeviceToHost,
+                                   c->stream));
+        les_note(c, hipEventRecord(c->ev_bounce[b], c->stream));
+    };
+    fetch(0, 0);
+    int b = 0;
+    for (long r0 = 0; r0 < rows; r0 += per, b ^= 1) {
+        const long n = std::min(per, rows - r0);
+        if (r0 + per < rows) fetch(r0 + per, b ^ 1);
+        les_note(c, hipEventSynchronize(c->ev_bounce[b]));
+        for (long r = 0; r < n; ++r)
+            std::memcpy(h + (size_t)(r0 + r) * (size_t)ld, c->bounce[b] + (size_t)r * nx, nx * 8);
+    }
+}
+
 // ---- scratch of the allocation-free entry point -----------------------------
 // les_zero_padding_noalloc keeps the x-padded intermediate of zero_padding in
 // this array instead of context memory.  Every GPU the library runs on holds
@@ -1009,6 +1113,10 @@ int les_destroy(les_ctx* c) {
     lin_destroy(c);
     for (void* p : c->allocs) (void)hipFree(p);
     if (c->cfl_host) (void)hipHostFree(c->cfl_host);
+    for (int i = 0; i < 2; ++i) {
+        if (c->bounce[i]) (void)hipHostFree(c->bounce[i]);
+        if (c->ev_bounce[i]) (void)hipEventDestroy(c->ev_bounce[i]);
+    }
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
     if (c->ev_join) (void)hipEventDestroy(c->ev_join);
     if (c->ev_obk) (void)hipEventDestroy(c->ev_obk);
@@ -1106,8 +1214,7 @@ int les_set_field(les_ctx* c, int id, const double* h, int ld, int lev0, int nle
         d = surf(c, id);
         if (!d || lev0 != 0 || nlev != 1) return LES_E_BADARG;
     }
-    les_note(c, hipMemcpy2DAsync(d, (size_t)c->nx * 8, h, (size_t)ld * 8, (size_t)c->nx * 8, (size_t)nlev * c->ny,
-                     hipMemcpyHostToDevice, c->stream));
+    rows_h2d(c, d, h, ld, (long)nlev * c->ny);
     if (df) convert(c->stream, df, (const double*)d, (long)nlev * (long)c->plane);
     return finish(c);
 }
@@ -1128,8 +1235,7 @@ int les_get_field(les_ctx* c, int id, double* h, int ld, int lev0, int nlev) {
         d = surf(c, id);
         if (!d || lev0 != 0 || nlev != 1) return LES_E_BADARG;
     }
-    les_note(c, hipMemcpy2DAsync(h, (size_t)ld * 8, d, (size_t)c->nx * 8, (size_t)c->nx * 8, (size_t)nlev * c->ny,
-                     hipMemcpyDeviceToHost, c->stream));
+    rows_d2h(c, h, d, ld, (long)nlev * c->ny);
     return finish(c);
 }
 
@@ -1200,8 +1306,7 @@ int les_test_filter(les_ctx* c, int f, int level, int which) {
 int les_fftn(les_ctx* c, const double* in, int ld, double* out_c) {
     if (!c || !in || !out_c || ld < c->nx) return LES_E_BADARG;
     double* w = c->work3[7];
-    les_note(c, hipMemcpy2DAsync(w, (size_t)c->nx * 8, in, (size_t)ld * 8, (size_t)c->nx * 8, c->ny, hipMemcpyHostToDevice,
-                     c->stream));
+    rows_h2d(c, w, in, ld, c->ny);
     cx<double>* sp = c->spec3[2];
     x_r2c<double>(c->stream, w, sp, c->ny, c->nx, c->lhx, c->tw_x, 1.0);
     yline_spec<double>(c->stream, sp, sp, 1, c->lhx, (long)c->ns, c->tw_y, SP_FWD, nullptr);
@@ -1216,16 +1321,14 @@ int les_ifftn(les_ctx* c, const double* in_c, double* out, int ld) {
     yline_spec<double>(c->stream, sp, sp, 1, c->lhx, (long)c->ns, c->tw_y, SP_INV, nullptr);
     double* w = c->work3[7];
     x_c2r<double>(c->stream, sp, w, c->ny, c->lhx, c->nx, c->tw_x, 0, 0.0);
-    les_note(c, hipMemcpy2DAsync(out, (size_t)ld * 8, w, (size_t)c->nx * 8, (size_t)c->nx * 8, c->ny, hipMemcpyDeviceToHost,
-                     c->stream));
+    rows_d2h(c, out, w, ld, c->ny);
     return finish(c);
 }
 
 int les_zero_padding(les_ctx* c, const double* var, int ld, double* big) {
     if (!c || !var || !big || ld < c->nx) return LES_E_BADARG;
     double* w = c->work3[7];
-    les_note(c, hipMemcpy2DAsync(w, (size_t)c->nx * 8, var, (size_t)ld * 8, (size_t)c->nx * 8, c->ny, hipMemcpyHostToDevice,
-                     c->stream));
+    rows_h2d(c, w, var, ld, c->ny);
     pad_f<double, double>(c, w, c->big3[0], 1);
     les_note(c, hipMemcpyAsync(big, c->big3[0], c->plane2 * 8, hipMemcpyDeviceToHost, c->stream));
     return finish(c);
@@ -1249,8 +1352,7 @@ int les_zero_unpadding(les_ctx* c, const double* big, double* var, int ld) {
     les_note(c, hipMemcpyAsync(c->big3[0], big, c->plane2 * 8, hipMemcpyHostToDevice, c->stream));
     double* w = c->work3[7];
     unpad_f<double>(c, c->big3[0], w, 1);
-    les_note(c, hipMemcpy2DAsync(var, (size_t)ld * 8, w, (size_t)c->nx * 8, (size_t)c->nx * 8, c->ny, hipMemcpyDeviceToHost,
-                     c->stream));
+    rows_d2h(c, var, w, ld, c->ny);
     return finish(c);
 }
 

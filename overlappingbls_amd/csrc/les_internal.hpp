@@ -141,6 +141,10 @@ struct les_ctx {
     hipError_t err;            // first asynchronous HIP error since the last finish()
     std::vector<void*> allocs;
     std::vector<les::Binding> binds;
+    // page-locked chunks of the strided host transfers (rows_h2d, rows_d2h),
+    // allocated on the first one; an event marks each chunk's last copy
+    double* bounce[2];
+    hipEvent_t ev_bounce[2];
 };
 
 // Record the first failing HIP runtime call of a context.

@@ -755,8 +755,7 @@ int les_lin_set(les_ctx* c, int id, const double* h, int ld, int lev0, int nlev)
         return LES_E_BADARG;
     if (lin_alloc(c) != hipSuccess) return LES_E_NOMEM;
     double* d = c->lin->b.v[v] + (pl ? 0 : (size_t)lev0 * c->plane);
-    les_note(c, hipMemcpy2DAsync(d, (size_t)c->nx * 8, h, (size_t)ld * 8, (size_t)c->nx * 8, (size_t)nlev * c->ny,
-                                 hipMemcpyHostToDevice, c->stream));
+    rows_h2d(c, d, h, ld, (long)nlev * c->ny);
     return finish(c);
 }
 
@@ -768,8 +767,7 @@ int les_lin_get(les_ctx* c, int id, double* h, int ld, int lev0, int nlev) {
         return LES_E_BADARG;
     if (lin_alloc(c) != hipSuccess) return LES_E_NOMEM;
     const double* d = c->lin->b.v[v] + (pl ? 0 : (size_t)lev0 * c->plane);
-    les_note(c, hipMemcpy2DAsync(h, (size_t)ld * 8, d, (size_t)c->nx * 8, (size_t)c->nx * 8, (size_t)nlev * c->ny,
-                                 hipMemcpyDeviceToHost, c->stream));
+    rows_d2h(c, h, d, ld, (long)nlev * c->ny);
     return finish(c);
 }
 

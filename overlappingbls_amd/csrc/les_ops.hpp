@@ -79,6 +79,12 @@ inline void test_filter_f(les_ctx* c, T* p, int nplanes, const double* G) {
     x_c2r<T>(c->stream, sp, p, (long)nplanes * c->ny, c->lhx, c->nx, c->tw_x, 0, 0.0);
 }
 
+// Host block (rows of nx values, row stride ld) to / from contiguous device
+// rows, enqueued on the context's stream (les_api.hip); a strided block in
+// pageable memory is complete on return.
+void rows_h2d(les_ctx* c, double* d, const double* h, int ld, long rows);
+void rows_d2h(les_ctx* c, double* h, const double* d, int ld, long rows);
+
 // Wait for both streams and return the first HIP error since the last call.
 int finish(les_ctx* c);
 
