@@ -11,6 +11,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "_lib")
 LIB = os.path.join(LIBDIR, "liblesgpu.so")
 SOURCES = [
+    "k_rg_g.hip", "k_rg_f.hip", "k_rg_e.hip", "k_rg_d.hip", "k_rg_c.hip", "k_rg_b.hip", "k_rg_a.hip",
     "k_lines.hip", "k_lines_rg.hip", "k_tdma.hip", "k_point.hip", "k_stats.hip", "k_lin.hip", "les_api.hip",
     "les_lin.hip", "les_files.hip", "les_prof.hip",
 ]
@@ -27,7 +28,7 @@ FLAGS = [
 ]
 
 
-def build(verbose: bool = False, jobs: int = 4) -> str:
+def build(verbose: bool = False, jobs: int = 8) -> str:
     """Compile every .hip source and link liblesgpu.so (always recompiles)."""
     os.makedirs(LIBDIR, exist_ok=True)
     objdir = os.path.join(LIBDIR, "obj")

@@ -198,26 +198,37 @@ __device__ __forceinline__ void dft(cx<T>* x) {
 // layout (the spectral multiplier of a same-length op stays in registers).
 constexpr int rg_nst(int n) {
     switch (n) {
-        case 512: case 768: return 3;
+        case 512: case 576: case 768: return 3;
         default: return 2;
     }
 }
 constexpr int rg_radix(int n, int s) {
     switch (n) {
+        case 16: return 4;
+        case 24: return s == 0 ? 4 : 6;
         case 32: return s == 0 ? 8 : 4;
+        case 36: return 6;
+        case 48: return s == 0 ? 6 : 8;
+        case 54: return s == 0 ? 6 : 9;
         case 64: return 8;
+        case 72: return s == 0 ? 8 : 9;
         case 96: return s == 0 ? 8 : 12;
+        case 108: return s == 0 ? 9 : 12;
         case 128: return s == 0 ? 16 : 8;
+        case 144: return 12;
+        case 162: return s == 0 ? 9 : 18;
         case 192: return s == 0 ? 16 : 12;
+        case 216: return s == 0 ? 12 : 18;
         case 256: return 16;
+        case 288: return s == 0 ? 16 : 18;
+        case 324: return 18;
         case 384: return s == 0 ? 16 : 24;
+        case 432: return s == 0 ? 18 : 24;
         case 512: return 8;
+        case 576: return s == 0 ? 9 : 8;
         case 768: return s == 0 ? 12 : 8;
         default: return 0;
     }
-}
-constexpr bool rg_supported(int n) {
-    return n == 64 || n == 96 || n == 128 || n == 192 || n == 256 || n == 384 || n == 512 || n == 768;
 }
 // radix of stage s of the transform in direction SIGN (inverse = reversed plan)
 constexpr int rg_r(int n, int s, int sign) { return sign < 0 ? rg_radix(n, s) : rg_radix(n, rg_nst(n) - 1 - s); }
