@@ -303,43 +303,47 @@ static int line_fam(LineOp op, bool y) {
 }
 
 template <typename T, typename TI>
-void xline_real(hipStream_t s, const TI* in, T* out, long nrows, int ld_in, int ld_out, const Twiddle& tin,
+void xline_real(hipStream_t s, const Batch<T, TI>& io, long nrows, int ld_in, int ld_out, const Twiddle& tin,
                 const Twiddle& tout, LineOp op, double kfac) {
-    FamScope fs(s, line_fam(op, false), (double)nrows * ((double)tin.n * sizeof(TI) + (double)tout.n * sizeof(T)));
-    if (g_use_ct && xline_real_ct<T, TI>(s, in, out, nrows, ld_in, ld_out, tin, tout, op, kfac)) return;
+    FamScope fs(s, line_fam(op, false), (double)io.nf * nrows * ((double)tin.n * sizeof(TI) + (double)tout.n * sizeof(T)));
+    if (g_use_ct && xline_real_ct<T, TI>(s, io, nrows, ld_in, ld_out, tin, tout, op, kfac)) return;
     const int L = tin.n > tout.n ? tin.n : tout.n;
     const int P = lines_per_block(L);
     const long nb = (nrows + 2 * P - 1) / (2 * P);
     const size_t lds = sizeof(cx<T>) * ((size_t)P * L + tin.n + tout.n);
-    hipLaunchKernelGGL((k_xline_real<T, TI>), dim3((unsigned)nb), dim3(NT), lds, s, in, out, nrows, ld_in, ld_out,
-                       tin.plan, tout.plan, twp<T>(tin), twp<T>(tout), (int)op, (T)kfac, P);
+    for (int f = 0; f < io.nf; ++f)
+        hipLaunchKernelGGL((k_xline_real<T, TI>), dim3((unsigned)nb), dim3(NT), lds, s, io.in[f], io.out[f], nrows,
+                           ld_in, ld_out, tin.plan, tout.plan, twp<T>(tin), twp<T>(tout), (int)op, (T)kfac, P);
 }
 
 template <typename T, typename TI>
-void yline_real(hipStream_t s, const TI* in, T* out, int nplanes, int ncols, int ld_in, int ld_out, long ps_in,
+void yline_real(hipStream_t s, const Batch<T, TI>& io, int nplanes, int ncols, int ld_in, int ld_out, long ps_in,
                 long ps_out, const Twiddle& tin, const Twiddle& tout, LineOp op, double kfac) {
     FamScope fs(s, line_fam(op, true),
-                (double)nplanes * ncols * ((double)tin.n * sizeof(TI) + (double)tout.n * sizeof(T)));
-    if (g_use_ct && yline_real_ct<T, TI>(s, in, out, nplanes, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, op, kfac)) return;
+                (double)io.nf * nplanes * ncols * ((double)tin.n * sizeof(TI) + (double)tout.n * sizeof(T)));
+    if (g_use_ct && yline_real_ct<T, TI>(s, io, nplanes, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, op, kfac)) return;
     const int L = tin.n > tout.n ? tin.n : tout.n;
     const int C = lines_per_block(L);
     const int nbx = (ncols + 2 * C - 1) / (2 * C);
     const size_t lds = sizeof(cx<T>) * ((size_t)C * L + tin.n + tout.n);
-    hipLaunchKernelGGL((k_yline_real<T, TI>), dim3(nbx, nplanes), dim3(NT), lds, s, in, out, ncols, ld_in, ld_out, ps_in,
-                       ps_out, tin.plan, tout.plan, twp<T>(tin), twp<T>(tout), (int)op, (T)kfac, C);
+    for (int f = 0; f < io.nf; ++f)
+        hipLaunchKernelGGL((k_yline_real<T, TI>), dim3(nbx, nplanes), dim3(NT), lds, s, io.in[f], io.out[f], ncols,
+                           ld_in, ld_out, ps_in, ps_out, tin.plan, tout.plan, twp<T>(tin), twp<T>(tout), (int)op,
+                           (T)kfac, C);
 }
 
 template <typename T, typename TI>
-void x_r2c(hipStream_t s, const TI* in, cx<T>* out, long nrows, int ld_in, int ldc, const Twiddle& tw,
+void x_r2c(hipStream_t s, const Batch<cx<T>, TI>& io, long nrows, int ld_in, int ldc, const Twiddle& tw,
            double scale, int kst) {
     if (kst < 0) kst = tw.n / 2 + 1;
-    FamScope fs(s, FAM_XR2C, (double)nrows * ((double)tw.n * sizeof(TI) + 2.0 * kst * sizeof(T)));
-    if (g_use_ct && x_r2c_ct<T, TI>(s, in, out, nrows, ld_in, ldc, tw, scale, kst)) return;
+    FamScope fs(s, FAM_XR2C, (double)io.nf * nrows * ((double)tw.n * sizeof(TI) + 2.0 * kst * sizeof(T)));
+    if (g_use_ct && x_r2c_ct<T, TI>(s, io, nrows, ld_in, ldc, tw, scale, kst)) return;
     const int P = lines_per_block(tw.n);
     const long nb = (nrows + 2 * P - 1) / (2 * P);
     const size_t lds = sizeof(cx<T>) * ((size_t)P * tw.n + tw.n);
-    hipLaunchKernelGGL((k_x_r2c<T, TI>), dim3((unsigned)nb), dim3(NT), lds, s, in, out, nrows, ld_in, ldc, tw.plan,
-                       twp<T>(tw), (T)scale, P, kst);
+    for (int f = 0; f < io.nf; ++f)
+        hipLaunchKernelGGL((k_x_r2c<T, TI>), dim3((unsigned)nb), dim3(NT), lds, s, io.in[f], io.out[f], nrows, ld_in,
+                           ldc, tw.plan, twp<T>(tw), (T)scale, P, kst);
 }
 
 template <typename T>
@@ -356,7 +360,7 @@ void x_c2r(hipStream_t s, const cx<T>* in, T* out, long nrows, int ldc, int ld_o
 }
 
 template <typename T>
-void yline_spec(hipStream_t s, const cx<T>* in, cx<T>* out, int nplanes, int ncols, long ps, const Twiddle& tw,
+void yline_spec(hipStream_t s, const Batch<cx<T>, cx<T>>& io, int nplanes, int ncols, long ps, const Twiddle& tw,
                 SpecOp op, const double* G, int ld, int ldG, int mc) {
     if (ld < 0) ld = ncols;
     if (ldG < 0) ldG = ld;
@@ -365,21 +369,22 @@ void yline_spec(hipStream_t s, const cx<T>* in, cx<T>* out, int nplanes, int nco
     // multiply-inverse reads, only the rows inside the filter support
     const double kept = (2 * mc - 1 < tw.n) ? (double)(2 * mc - 1) : (double)tw.n;
     const double rin = (op == SP_MULINV) ? kept : (double)tw.n, rout = (op == SP_FWD) ? kept : (double)tw.n;
-    FamScope fs(s, FAM_YSPEC, (double)nplanes * ncols * 2.0 * sizeof(T) * (rin + rout));
-    if (g_use_ct && yline_spec_ct<T>(s, in, out, nplanes, ncols, ps, tw, op, G, ld, ldG, mc)) return;
+    FamScope fs(s, FAM_YSPEC, (double)io.nf * nplanes * ncols * 2.0 * sizeof(T) * (rin + rout));
+    if (g_use_ct && yline_spec_ct<T>(s, io, nplanes, ncols, ps, tw, op, G, ld, ldG, mc)) return;
     const int C = lines_per_block(tw.n);
     const int nbx = (ncols + C - 1) / C;
     const size_t lds = sizeof(cx<T>) * ((size_t)C * tw.n + tw.n);
-    hipLaunchKernelGGL(k_yline_spec<T>, dim3(nbx, nplanes), dim3(NT), lds, s, in, out, ncols, ld, ldG, mc, ps,
-                       tw.plan, twp<T>(tw), (int)op, G, C);
+    for (int f = 0; f < io.nf; ++f)
+        hipLaunchKernelGGL(k_yline_spec<T>, dim3(nbx, nplanes), dim3(NT), lds, s, io.in[f], io.out[f], ncols, ld, ldG,
+                           mc, ps, tw.plan, twp<T>(tw), (int)op, G, C);
 }
 
 #define LES_INST_LINES(T, TI)                                                                                   \
-    template void xline_real<T, TI>(hipStream_t, const TI*, T*, long, int, int, const Twiddle&, const Twiddle&,      \
+    template void xline_real<T, TI>(hipStream_t, const Batch<T, TI>&, long, int, int, const Twiddle&, const Twiddle&,      \
                                     LineOp, double);                                                               \
-    template void yline_real<T, TI>(hipStream_t, const TI*, T*, int, int, int, int, long, long, const Twiddle&,      \
+    template void yline_real<T, TI>(hipStream_t, const Batch<T, TI>&, int, int, int, int, long, long, const Twiddle&,      \
                                     const Twiddle&, LineOp, double);                                               \
-    template void x_r2c<T, TI>(hipStream_t, const TI*, cx<T>*, long, int, int, const Twiddle&, double, int);
+    template void x_r2c<T, TI>(hipStream_t, const Batch<cx<T>, TI>&, long, int, int, const Twiddle&, double, int);
 LES_INST_LINES(double, double)
 LES_INST_LINES(float, float)
 LES_INST_LINES(float, double)
@@ -387,9 +392,9 @@ LES_INST_LINES(float, double)
 template void x_c2r<double>(hipStream_t, const cx<double>*, double*, long, int, int, const Twiddle&, int, double,
                             int);
 template void x_c2r<float>(hipStream_t, const cx<float>*, float*, long, int, int, const Twiddle&, int, double, int);
-template void yline_spec<double>(hipStream_t, const cx<double>*, cx<double>*, int, int, long, const Twiddle&,
+template void yline_spec<double>(hipStream_t, const Batch<cx<double>, cx<double>>&, int, int, long, const Twiddle&,
                                  SpecOp, const double*, int, int, int);
-template void yline_spec<float>(hipStream_t, const cx<float>*, cx<float>*, int, int, long, const Twiddle&,
+template void yline_spec<float>(hipStream_t, const Batch<cx<float>, cx<float>>&, int, int, long, const Twiddle&,
                                 SpecOp, const double*, int, int, int);
 
 }  // namespace les

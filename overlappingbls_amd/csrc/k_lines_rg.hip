@@ -58,24 +58,25 @@ static bool pairs_aligned(const TI* in, const T* out, int ncols, int ld_in, int 
 }
 
 template <typename T, typename TI>
-bool xline_real_ct(hipStream_t s, const TI* in, T* out, long nrows, int ld_in, int ld_out, const Twiddle& tin,
+bool xline_real_ct(hipStream_t s, const Batch<T, TI>& io, long nrows, int ld_in, int ld_out, const Twiddle& tin,
                    const Twiddle& tout, LineOp op, double kfac) {
     const RgTable* t = rg_table(rg_length(tin, tout, op));
-    return t && rg_io<T, TI>(t).x(s, op, in, out, nrows, ld_in, ld_out, tin, tout, kfac);
+    return t && rg_io<T, TI>(t).x(s, op, io, nrows, ld_in, ld_out, tin, tout, kfac);
 }
 template <typename T, typename TI>
-bool yline_real_ct(hipStream_t s, const TI* in, T* out, int nplanes, int ncols, int ld_in, int ld_out, long ps_in,
+bool yline_real_ct(hipStream_t s, const Batch<T, TI>& io, int nplanes, int ncols, int ld_in, int ld_out, long ps_in,
                    long ps_out, const Twiddle& tin, const Twiddle& tout, LineOp op, double kfac) {
-    if (!pairs_aligned(in, out, ncols, ld_in, ld_out, ps_in, ps_out)) return false;
+    for (int f = 0; f < io.nf; ++f)
+        if (!pairs_aligned(io.in[f], io.out[f], ncols, ld_in, ld_out, ps_in, ps_out)) return false;
     const RgTable* t = rg_table(rg_length(tin, tout, op));
-    return t && rg_io<T, TI>(t).y(s, op, in, out, nplanes, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, kfac);
+    return t && rg_io<T, TI>(t).y(s, op, io, nplanes, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, kfac);
 }
 template <typename T, typename TI>
-bool x_r2c_ct(hipStream_t s, const TI* in, cx<T>* out, long nrows, int ld_in, int ldc, const Twiddle& tw,
+bool x_r2c_ct(hipStream_t s, const Batch<cx<T>, TI>& io, long nrows, int ld_in, int ldc, const Twiddle& tw,
               double scale, int kst) {
     const RgTable* t = rg_table(tw.n);
     if (!t) return false;
-    rg_io<T, TI>(t).r2c(s, in, out, nrows, ld_in, ldc, tw, scale, kst);
+    rg_io<T, TI>(t).r2c(s, io, nrows, ld_in, ldc, tw, scale, kst);
     return true;
 }
 template <typename T>
@@ -87,11 +88,11 @@ bool x_c2r_ct(hipStream_t s, const cx<T>* in, T* out, long nrows, int ldc, int l
     return true;
 }
 template <typename T>
-bool yline_spec_ct(hipStream_t s, const cx<T>* in, cx<T>* out, int nplanes, int ncols, long ps, const Twiddle& tw,
+bool yline_spec_ct(hipStream_t s, const Batch<cx<T>, cx<T>>& io, int nplanes, int ncols, long ps, const Twiddle& tw,
                    SpecOp op, const double* G, int ld, int ldG, int mc) {
     const RgTable* t = rg_table(tw.n);
     if (!t) return false;
-    rg_ops<T>(t).spec(s, op, in, out, nplanes, ncols, ps, tw, G, ld, ldG, mc);
+    rg_ops<T>(t).spec(s, op, io, nplanes, ncols, ps, tw, G, ld, ldG, mc);
     return true;
 }
 
@@ -143,11 +144,11 @@ template bool vort_pad_x<float>(hipStream_t, const VortIn<float>&, float*, float
                                 const Twiddle&);
 
 #define INST_IO(T, TI)                                                                                       \
-    template bool xline_real_ct<T, TI>(hipStream_t, const TI*, T*, long, int, int, const Twiddle&, const Twiddle&, \
+    template bool xline_real_ct<T, TI>(hipStream_t, const Batch<T, TI>&, long, int, int, const Twiddle&, const Twiddle&, \
                                        LineOp, double);                                                          \
-    template bool yline_real_ct<T, TI>(hipStream_t, const TI*, T*, int, int, int, int, long, long, const Twiddle&, \
+    template bool yline_real_ct<T, TI>(hipStream_t, const Batch<T, TI>&, int, int, int, int, long, long, const Twiddle&, \
                                        const Twiddle&, LineOp, double);                                          \
-    template bool x_r2c_ct<T, TI>(hipStream_t, const TI*, cx<T>*, long, int, int, const Twiddle&, double, int);
+    template bool x_r2c_ct<T, TI>(hipStream_t, const Batch<cx<T>, TI>&, long, int, int, const Twiddle&, double, int);
 INST_IO(double, double)
 INST_IO(float, float)
 INST_IO(float, double)
@@ -156,9 +157,9 @@ template bool x_c2r_ct<double>(hipStream_t, const cx<double>*, double*, long, in
                                int);
 template bool x_c2r_ct<float>(hipStream_t, const cx<float>*, float*, long, int, int, const Twiddle&, int, double,
                               int);
-template bool yline_spec_ct<double>(hipStream_t, const cx<double>*, cx<double>*, int, int, long, const Twiddle&,
+template bool yline_spec_ct<double>(hipStream_t, const Batch<cx<double>, cx<double>>&, int, int, long, const Twiddle&,
                                     SpecOp, const double*, int, int, int);
-template bool yline_spec_ct<float>(hipStream_t, const cx<float>*, cx<float>*, int, int, long, const Twiddle&,
+template bool yline_spec_ct<float>(hipStream_t, const Batch<cx<float>, cx<float>>&, int, int, long, const Twiddle&,
                                    SpecOp, const double*, int, int, int);
 
 }  // namespace les

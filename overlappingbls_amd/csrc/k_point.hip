@@ -889,24 +889,56 @@ void ddz_w_dev(les_ctx* c, W* d, const TI* f) {
     hipLaunchKernelGGL((k_ddz_w<W, TI>), grid_for(p.plane * (p.nz + 1)), dim3(256), 0, c->stream, d, f, p);
 }
 
+// ddz_uv of u and v and ddz_w of w in one launch (component blockIdx.y)
+template <typename W>
+__global__ void k_ddz_uvw(W* uz, W* vz, W* wz, const double* __restrict__ u, const double* __restrict__ v,
+                          const double* __restrict__ w, KP p) {
+    const long n = p.plane * (p.nz + 1);
+    const double cst = 1.0 / p.dz;
+    const int m = blockIdx.y;
+    W* d = m == 0 ? uz : (m == 1 ? vz : wz);
+    const double* __restrict__ f = m == 0 ? u : (m == 1 ? v : w);
+    GRID_LOOP(i, n) {
+        const int k = (int)(i / p.plane);
+        if (k == 0) d[i] = BOGUS;
+        else if (m < 2) {
+            if (k >= 2 && k <= p.nz - 1) d[i] = cst * (f[i] - f[i - p.plane]);
+        } else if (k == p.nz) d[i] = 0.0;
+        else d[i] = cst * (f[i + p.plane] - f[i]);
+    }
+}
+
+template <typename W>
+void ddz_uvw_dev(les_ctx* c) {
+    FamScope fs(c->stream, FAM_DDZ, 3.0 * (double)(8 + sizeof(W)) * (double)c->plane * (double)c->nlev);
+    KP p = kp(c);
+    dim3 g = grid_for(p.plane * (p.nz + 1));
+    g.y = 3;
+    hipLaunchKernelGGL(k_ddz_uvw<W>, g, dim3(256), 0, c->stream, WF<W>(c, LES_F_DUDZ), WF<W>(c, LES_F_DVDZ),
+                       WF<W>(c, LES_F_DWDZ), (const double*)c->f3[LES_F_U], (const double*)c->f3[LES_F_V],
+                       (const double*)c->f3[LES_F_W], p);
+}
+
 // ---- divstress, 107_divstress.f90:36-102 ---------------------------------------
 // a = d/dx tx, b = d/dy ty, f = tz (FD taken here: ddz_w for uv, ddz_uv for w)
 template <typename W>
+__device__ __forceinline__ void divstress_at(W* out, const W* __restrict__ a, const W* __restrict__ b,
+                                             const W* __restrict__ f, const KP& p, int wver, double cst, long i) {
+    const int k = (int)(i / p.plane);
+    if (!wver) {
+        if (k == 0 || k == p.nz) out[i] = BOGUS;
+        else out[i] = (double)a[i] + (double)b[i] + cst * ((double)f[i + p.plane] - (double)f[i]);
+    } else {
+        if (k == 0) out[i] = BOGUS;
+        else if (k == 1 || k == p.nz) out[i] = (double)a[i] + (double)b[i];
+        else out[i] = (double)a[i] + (double)b[i] + cst * ((double)f[i] - (double)f[i - p.plane]);
+    }
+}
+template <typename W>
 __global__ void k_divstress(W* out, const W* __restrict__ a, const W* __restrict__ b, const W* __restrict__ f, KP p,
                             int wver) {
-    const long n = p.plane * (p.nz + 1);
     const double cst = 1.0 / p.dz;
-    GRID_LOOP(i, n) {
-        const int k = (int)(i / p.plane);
-        if (!wver) {
-            if (k == 0 || k == p.nz) out[i] = BOGUS;
-            else out[i] = (double)a[i] + (double)b[i] + cst * ((double)f[i + p.plane] - (double)f[i]);
-        } else {
-            if (k == 0) out[i] = BOGUS;
-            else if (k == 1 || k == p.nz) out[i] = (double)a[i] + (double)b[i];
-            else out[i] = (double)a[i] + (double)b[i] + cst * ((double)f[i] - (double)f[i - p.plane]);
-        }
-    }
+    GRID_LOOP(i, p.plane * (p.nz + 1)) divstress_at<W>(out, a, b, f, p, wver, cst, i);
 }
 
 template <typename W>
@@ -914,6 +946,40 @@ void divstress_combine_dev(les_ctx* c, W* out, const W* a, const W* b, const W* 
     FamScope fs(c->stream, FAM_DIVSTRESS, 4.0 * sizeof(W) * (double)c->plane * (double)c->nlev);
     KP p = kp(c);
     hipLaunchKernelGGL(k_divstress<W>, grid_for(p.plane * (p.nz + 1)), dim3(256), 0, c->stream, out, a, b, d, p, wver);
+}
+
+// the step's three divergences in one launch (component blockIdx.y: x, y
+// divstress_uv, z divstress_w)
+template <typename W>
+struct Div3 {
+    W* out[3];
+    const W *a[3], *b[3], *f[3];
+};
+template <typename W>
+__global__ void k_divstress3(Div3<W> d, KP p) {
+    const double cst = 1.0 / p.dz;
+    const int m = blockIdx.y;
+    W* out = m == 0 ? d.out[0] : (m == 1 ? d.out[1] : d.out[2]);
+    const W* __restrict__ a = m == 0 ? d.a[0] : (m == 1 ? d.a[1] : d.a[2]);
+    const W* __restrict__ b = m == 0 ? d.b[0] : (m == 1 ? d.b[1] : d.b[2]);
+    const W* __restrict__ f = m == 0 ? d.f[0] : (m == 1 ? d.f[1] : d.f[2]);
+    GRID_LOOP(i, p.plane * (p.nz + 1)) divstress_at<W>(out, a, b, f, p, m == 2, cst, i);
+}
+
+template <typename W>
+void divstress_combine3_dev(les_ctx* c, W* const a[3], W* const b[3]) {
+    FamScope fs(c->stream, FAM_DIVSTRESS, 12.0 * sizeof(W) * (double)c->plane * (double)c->nlev);
+    KP p = kp(c);
+    Div3<W> d;
+    for (int m = 0; m < 3; ++m) {
+        d.out[m] = WF<W>(c, LES_F_DIVTX + m);
+        d.a[m] = a[m];
+        d.b[m] = b[m];
+        d.f[m] = WF<W>(c, m == 0 ? LES_F_TXZ : (m == 1 ? LES_F_TYZ : LES_F_TZZ));
+    }
+    dim3 g = grid_for(p.plane * (p.nz + 1));
+    g.y = 3;
+    hipLaunchKernelGGL(k_divstress3<W>, g, dim3(256), 0, c->stream, d, p);
 }
 
 // ---- convec, 108_convec.f90:44-69 and cross_product :103-202 -------------------
@@ -1688,6 +1754,8 @@ void max3_dev(les_ctx* c, double* out, bool lag) {
     template void strain_stress_dev<W>(les_ctx*);                                                           \
     template void lagrange_prep_dev<W>(les_ctx*, W*);                                                       \
     template void lagrange_contract_dev<W>(les_ctx*, const W*, const W*, int, int);                         \
+    template void ddz_uvw_dev<W>(les_ctx*);                                                                 \
+    template void divstress_combine3_dev<W>(les_ctx*, W* const[3], W* const[3]);                            \
     template void divstress_combine_dev<W>(les_ctx*, W*, const W*, const W*, const W*, int);                \
     template void vorticity_dev<W>(les_ctx*, W*, W*, W*);                                                   \
     template void cross_product_dev<W>(les_ctx*, const W*, const W*, const W*, W*, W*, W*);                 \

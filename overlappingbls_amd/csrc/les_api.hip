@@ -30,12 +30,9 @@ void press_solve(les_ctx* c, const double* u, const double* v, const double* w, 
     press_rhs_prep_on<W>(c, rx, ry, rz, u, v, w, divtz, modi);
     cx<W>*Hx = scr<W>(c->spec3[0]), *Hy = scr<W>(c->spec3[1]), *Hz = scr<W>(c->spec3[2]);
     const long rows = (long)(nz + 1) * c->ny;
-    x_r2c<W>(c->stream, rx, Hx, rows, c->nx, c->lhx, c->tw_x, 1.0);
-    x_r2c<W>(c->stream, ry, Hy, rows, c->nx, c->lhx, c->tw_x, 1.0);
-    x_r2c<W>(c->stream, rz, Hz, rows, c->nx, c->lhx, c->tw_x, 1.0);
-    yline_spec<W>(c->stream, Hx, Hx, nz + 1, c->lhx, (long)ns, c->tw_y, SP_FWD, nullptr);
-    yline_spec<W>(c->stream, Hy, Hy, nz + 1, c->lhx, (long)ns, c->tw_y, SP_FWD, nullptr);
-    yline_spec<W>(c->stream, Hz, Hz, nz + 1, c->lhx, (long)ns, c->tw_y, SP_FWD, nullptr);
+    x_r2c<W, W>(c->stream, batch3<cx<W>, W>(rx, ry, rz, Hx, Hy, Hz), rows, c->nx, c->lhx, c->tw_x, 1.0);
+    yline_spec<W>(c->stream, batch3<cx<W>, cx<W>>(Hx, Hy, Hz, Hx, Hy, Hz), nz + 1, c->lhx, (long)ns, c->tw_y, SP_FWD,
+                  nullptr);
     cx<W>* ph;
     const double* hzm = nullptr;
     if (sizeof(W) == sizeof(double)) {
@@ -335,12 +332,13 @@ void wallstress(les_ctx* c, int top) {
         return;
     }
     const int lev = top ? c->nz - 1 : 1;
-    double* w = c->work3[7];  // two planes: u1, v1
-    les_note(c, hipMemcpyAsync(w, F(c, LES_F_U) + (size_t)lev * c->plane, c->plane * 8, hipMemcpyDeviceToDevice,
-                               c->stream));
-    les_note(c, hipMemcpyAsync(w + c->plane, F(c, LES_F_V) + (size_t)lev * c->plane, c->plane * 8,
-                               hipMemcpyDeviceToDevice, c->stream));
-    test_filter_f<double>(c, w, 2, c->Gtest);
+    double* w = c->work3[7];  // two planes: u1, v1, test-filtered
+    const size_t o = (size_t)lev * c->plane;
+    cx<double>* sp = c->spec3[2];
+    Batch<cx<double>, double> b{2, {F(c, LES_F_U) + o, F(c, LES_F_V) + o, nullptr}, {sp, sp + c->ns, nullptr}};
+    x_r2c<double, double>(c->stream, b, c->ny, c->nx, c->lhx, c->tw_x, 1.0);
+    yline_spec<double>(c->stream, sp, sp, 2, c->lhx, (long)c->ns, c->tw_y, SP_FILT, c->Gtest);
+    x_c2r<double>(c->stream, sp, w, 2L * c->ny, c->lhx, c->nx, c->tw_x, 0, 0.0);
     wallstress_dev<W>(c, top, w, w + c->plane);
 }
 
@@ -419,6 +417,22 @@ void divstress(les_ctx* c, W* out, const W* tx, const W* ty, const W* tz, int wv
     divstress_combine_dev<W>(c, out, a, b, tz, wver);
 }
 
+// the step's three divergences: divstress_uv of (txx, txy, txz) and (txy,
+// tyy, tyz), divstress_w of (txz, tyz, tzz), each pass one launch
+template <typename W>
+void divstress3(les_ctx* c) {
+    W *txx = WF<W>(c, LES_F_TXX), *txy = WF<W>(c, LES_F_TXY), *txz = WF<W>(c, LES_F_TXZ);
+    W *tyy = WF<W>(c, LES_F_TYY), *tyz = WF<W>(c, LES_F_TYZ), *tzz = WF<W>(c, LES_F_TZZ);
+    W *a[3], *b[3];
+    for (int m = 0; m < 3; ++m) {
+        a[m] = scr<W>(c->work3[m]);
+        b[m] = scr<W>(c->work3[3 + m]);
+    }
+    ddx3_f<W, W>(c, batch3<W, W>(txx, txy, txz, a[0], a[1], a[2]), 0, (int)c->nlev);
+    ddy3_f<W, W>(c, batch3<W, W>(txy, tyy, tyz, b[0], b[1], b[2]), 0, (int)c->nlev);
+    divstress_combine3_dev<W>(c, a, b);
+}
+
 template <typename W>
 void convec(les_ctx* c, bool uvw_on_aux = false) {
     const int nz = c->nz;
@@ -429,9 +443,8 @@ void convec(les_ctx* c, bool uvw_on_aux = false) {
     W* big[6];
     for (int i = 0; i < 6; ++i) big[i] = scr<W>(c->big3[i]);
     if (!uvw_on_aux) {
-        pad_f<W, double>(c, F(c, LES_F_U), ub, (int)c->nlev);
-        pad_f<W, double>(c, F(c, LES_F_V), vb, (int)c->nlev);
-        pad_f<W, double>(c, F(c, LES_F_W), wb, (int)c->nlev);
+        pad3_f<W, double>(c, batch3<W, double>(F(c, LES_F_U), F(c, LES_F_V), F(c, LES_F_W), ub, vb, wb),
+                          (int)c->nlev);
     }
     // vorticity and the x pass of its pads in one kernel (x-padded rows in
     // big[3..5]), then the y passes into big[0..2]
@@ -439,15 +452,12 @@ void convec(les_ctx* c, bool uvw_on_aux = false) {
                        WF<W>(c, LES_F_DVDZ), WF<W>(c, LES_F_DWDX), WF<W>(c, LES_F_DWDY)};
     const bool fz = c->fuse && g_use_ct;
     if (fz && vort_pad_x<W>(c->stream, vg, big[3], big[4], big[5], nz, c->ny, c->tw_x, c->tw_x2)) {
-        for (int m = 0; m < 3; ++m)
-            yline_real<W>(c->stream, big[3 + m], big[m] + np2, nz, c->nx2, c->nx2, c->nx2, (long)c->ny * c->nx2,
-                          (long)np2, c->tw_y, c->tw_y2, OP_PAD, 0.0);
+        yline_real<W>(c->stream, batch3<W, W>(big[3], big[4], big[5], big[0] + np2, big[1] + np2, big[2] + np2), nz,
+                      c->nx2, c->nx2, c->nx2, (long)c->ny * c->nx2, (long)np2, c->tw_y, c->tw_y2, OP_PAD, 0.0);
     } else {
         W *v1 = scr<W>(c->work3[2]), *v2 = scr<W>(c->work3[3]), *v3 = scr<W>(c->work3[4]);
         vorticity_dev<W>(c, v1, v2, v3);
-        pad_f<W, W>(c, v1 + np, big[0] + np2, nz);
-        pad_f<W, W>(c, v2 + np, big[1] + np2, nz);
-        pad_f<W, W>(c, v3 + np, big[2] + np2, nz);
+        pad3_f<W, W>(c, batch3<W, W>(v1 + np, v2 + np, v3 + np, big[0] + np2, big[1] + np2, big[2] + np2), nz);
     }
     W* cxf = WF<W>(c, LES_F_CX);
     W* cyf = WF<W>(c, LES_F_CY);
@@ -457,15 +467,11 @@ void convec(les_ctx* c, bool uvw_on_aux = false) {
     const ConvIn<W> ci{ub, vb, wb, big[0], big[1], big[2], c->ust, c->vst};
     if (uvw_on_aux) les_note(c, hipStreamWaitEvent(c->stream, c->ev_uvw, 0));
     if (fz && cross_unpad_x<W>(c->stream, ci, 0, big[3], big[4], big[5], nz, c->ny2, c->tw_x2, c->tw_x)) {
-        W* dst[3] = {cxf, cyf, czf};
-        for (int m = 0; m < 3; ++m)
-            yline_real<W>(c->stream, big[3 + m], dst[m] + np, nz - 1, c->nx, c->nx, c->nx, (long)c->ny2 * c->nx,
-                          (long)np, c->tw_y2, c->tw_y, OP_UNPAD, 0.0);
+        yline_real<W>(c->stream, batch3<W, W>(big[3], big[4], big[5], cxf + np, cyf + np, czf + np), nz - 1, c->nx,
+                      c->nx, c->nx, (long)c->ny2 * c->nx, (long)np, c->tw_y2, c->tw_y, OP_UNPAD, 0.0);
     } else {
         cross_product_dev<W>(c, big[0], big[1], big[2], big[3], big[4], big[5]);
-        unpad_f<W>(c, big[3] + np2, cxf + np, nz - 1);
-        unpad_f<W>(c, big[4] + np2, cyf + np, nz - 1);
-        unpad_f<W>(c, big[5] + np2, czf + np, nz - 1);
+        unpad3_f<W>(c, batch3<W, W>(big[3] + np2, big[4] + np2, big[5] + np2, cxf + np, cyf + np, czf + np), nz - 1);
     }
     fill_runs<W>(c->stream, (long)np, BOGUS, {cxf, cyf, czf, cxf + (size_t)nz * np, cyf + (size_t)nz * np});
 }
@@ -483,9 +489,10 @@ template <typename W>
 void theta_pads(les_ctx* c, W* dtdx, W* dtdy, W* dtdz) {
     const int nz = c->nz;
     const size_t np = c->plane, np2 = c->plane2;
-    pad_f<W, W>(c, dtdx + np, scr<W>(c->tbig[0]) + np2, nz - 1);
-    pad_f<W, W>(c, dtdy + np, scr<W>(c->tbig[1]) + np2, nz - 1);
-    pad_f<W, W>(c, dtdz + 2 * np, scr<W>(c->tbig[2]) + 2 * np2, nz - 1);
+    pad3_f<W, W>(c,
+                 batch3<W, W>(dtdx + np, dtdy + np, dtdz + 2 * np, scr<W>(c->tbig[0]) + np2, scr<W>(c->tbig[1]) + np2,
+                              scr<W>(c->tbig[2]) + 2 * np2),
+                 nz - 1);
 }
 
 // filter_data(theta), dTdx, dTdy, dTdz, the theta RHS history (:111-140) and
@@ -521,9 +528,10 @@ template <typename W>
 void uvw_pads_overlap(les_ctx* c) {
     std::swap(c->stream, c->aux);
     std::swap(c->work3[6], c->tscr[3]);
-    pad_f<W, double>(c, F(c, LES_F_U), scr<W>(c->u_big), (int)c->nlev);
-    pad_f<W, double>(c, F(c, LES_F_V), scr<W>(c->v_big), (int)c->nlev);
-    pad_f<W, double>(c, F(c, LES_F_W), scr<W>(c->w_big), (int)c->nlev);
+    pad3_f<W, double>(c,
+                      batch3<W, double>(F(c, LES_F_U), F(c, LES_F_V), F(c, LES_F_W), scr<W>(c->u_big),
+                                        scr<W>(c->v_big), scr<W>(c->w_big)),
+                      (int)c->nlev);
     les_note(c, hipEventRecord(c->ev_uvw, c->stream));
     std::swap(c->work3[6], c->tscr[3]);
     std::swap(c->stream, c->aux);
@@ -734,15 +742,13 @@ void step_body(les_ctx* c, int jt, Tape* tape = nullptr, bool stats = true) {
     if (ovl) uvw_pads_overlap<W>(c);             // convec's padded u, v, w on aux
     const int nl = (int)c->nlev;
     const double *u = F(c, LES_F_U), *v = F(c, LES_F_V), *w = F(c, LES_F_W);
-    ddx_f<W, double>(c, WF<W>(c, LES_F_DUDX), u, 0, nl);
-    ddy_f<W, double>(c, WF<W>(c, LES_F_DUDY), u, 0, nl);
-    ddx_f<W, double>(c, WF<W>(c, LES_F_DVDX), v, 0, nl);
-    ddy_f<W, double>(c, WF<W>(c, LES_F_DVDY), v, 0, nl);
-    ddx_f<W, double>(c, WF<W>(c, LES_F_DWDX), w, 0, nl);
-    ddy_f<W, double>(c, WF<W>(c, LES_F_DWDY), w, 0, nl);
-    ddz_uv_dev<W, double>(c, WF<W>(c, LES_F_DUDZ), u);
-    ddz_uv_dev<W, double>(c, WF<W>(c, LES_F_DVDZ), v);
-    ddz_w_dev<W, double>(c, WF<W>(c, LES_F_DWDZ), w);
+    ddx3_f<W, double>(c,
+                      batch3<W, double>(u, v, w, WF<W>(c, LES_F_DUDX), WF<W>(c, LES_F_DVDX), WF<W>(c, LES_F_DWDX)), 0,
+                      nl);
+    ddy3_f<W, double>(c,
+                      batch3<W, double>(u, v, w, WF<W>(c, LES_F_DUDY), WF<W>(c, LES_F_DVDY), WF<W>(c, LES_F_DWDY)), 0,
+                      nl);
+    ddz_uvw_dev<W>(c);
     // theta's filter, gradients and pads: on aux (submitted after the
     // derivatives, so that the host, which has a bounded number of launches
     // outstanding, hands the momentum stream its work first), or in order
@@ -755,11 +761,7 @@ void step_body(les_ctx* c, int jt, Tape* tape = nullptr, bool stats = true) {
     if (tape) tape_save(c, tape, TAPE_WALL);
     wallstress<W>(c, 1);
     sgs_stag<W>(c, jt, tape != nullptr || (stats && stats_step(c, jt)));
-    W *txx = WF<W>(c, LES_F_TXX), *txy = WF<W>(c, LES_F_TXY), *txz = WF<W>(c, LES_F_TXZ);
-    W *tyy = WF<W>(c, LES_F_TYY), *tyz = WF<W>(c, LES_F_TYZ), *tzz = WF<W>(c, LES_F_TZZ);
-    divstress<W>(c, WF<W>(c, LES_F_DIVTX), txx, txy, txz, 0);
-    divstress<W>(c, WF<W>(c, LES_F_DIVTY), txy, tyy, tyz, 0);
-    divstress<W>(c, WF<W>(c, LES_F_DIVTZ), txz, tyz, tzz, 1);
+    divstress3<W>(c);
     convec<W>(c, ovl);
     if (ovl) theta_post_overlap<W>(c, jt, tape);
     else theta_post<W>(c, jt, tape);
@@ -767,9 +769,7 @@ void step_body(les_ctx* c, int jt, Tape* tape = nullptr, bool stats = true) {
     press_stag_array<W>(c, jt);
     gradp_project_dev<W>(c, jt, !(ovl && theta_active(c, jt)));
     if (st) diagnostics_ke(c);
-    filter_f<double>(c, F(c, LES_F_U), 0, nl);
-    filter_f<double>(c, F(c, LES_F_V), 0, nl);
-    filter_f<double>(c, F(c, LES_F_W), 0, nl);
+    filter3_f(c, F(c, LES_F_U), F(c, LES_F_V), F(c, LES_F_W), nl);
     if (ovl) join(c);
     if (st) avg_slices<W>(c, jt);
     if (tape) tape_save(c, tape, TAPE_END);
@@ -1047,9 +1047,9 @@ int les_create(const les_params* prm, les_ctx** out) {
     for (int i = 0; i < 3 && e == hipSuccess; ++i) e = dalloc(c, &c->tbig[i], B3);
     if (e == hipSuccess) e = dalloc(c, &c->th_mean, c->nlev);
     if (e == hipSuccess) e = dalloc(c, &c->th1_copy, c->plane);
-    for (int i = 0; i < 8 && e == hipSuccess; ++i) e = dalloc(c, &c->work3[i], i == 6 ? (F3 * 3) / 2 + c->plane2 : F3);
+    for (int i = 0; i < 8 && e == hipSuccess; ++i) e = dalloc(c, &c->work3[i], i == 6 ? 3 * ((F3 * 3) / 2) + c->plane2 : F3);
     for (int i = 0; i < 3 && e == hipSuccess; ++i) e = dalloc(c, &c->tscr[i], F3);
-    if (e == hipSuccess) e = dalloc(c, &c->tscr[3], (F3 * 3) / 2 + c->plane2);
+    if (e == hipSuccess) e = dalloc(c, &c->tscr[3], 3 * ((F3 * 3) / 2) + c->plane2);
     if (e == hipSuccess) e = dalloc(c, &c->tscr[4], B3);
     for (int i = 0; i < 4 && e == hipSuccess; ++i) e = dalloc(c, &c->spec3[i], c->ns * c->nlev);
     const size_t np21 = (size_t)21 * c->nz;

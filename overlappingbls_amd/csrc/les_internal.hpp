@@ -184,20 +184,40 @@ struct FamScope {
 };
 
 // ---- line transforms (k_lines.hip) ---------------------------------------
+// Up to BATCH fields per launch: the same operation on each in[f] -> out[f].
+// The step transforms its fields in threes (u, v, w and their kin), and at
+// 64^3 and below a launch costs as much as its work: a 10-step window takes
+// 3.86 ms against 5.14 ms with one launch per field at 64^3, 15.6 against
+// 17.0 ms at 128^3, and the same at 256^3, where the passes are bound by HBM.
+constexpr int BATCH = 3;
+template <typename TO, typename TI>
+struct Batch {
+    int nf;
+    const TI* in[BATCH];
+    TO* out[BATCH];
+};
+template <typename TO, typename TI>
+inline Batch<TO, TI> batch1(const TI* in, TO* out) {
+    return {1, {in, in, in}, {out, out, out}};
+}
+template <typename TO, typename TI>
+inline Batch<TO, TI> batch3(const TI* a, const TI* b, const TI* c, TO* oa, TO* ob, TO* oc) {
+    return {3, {a, b, c}, {oa, ob, oc}};
+}
 // Real x-lines: nrows rows, row r at in + r*ld_in (length nin) -> out + r*ld_out.
 template <typename T, typename TI = T>
-void xline_real(hipStream_t s, const TI* in, T* out, long nrows, int ld_in, int ld_out,
+void xline_real(hipStream_t s, const Batch<T, TI>& io, long nrows, int ld_in, int ld_out,
                 const Twiddle& tin, const Twiddle& tout, LineOp op, double kfac);
 // Real y-lines on nplanes planes: (nin rows x ncols) -> (nout rows x ncols).
 template <typename T, typename TI = T>
-void yline_real(hipStream_t s, const TI* in, T* out, int nplanes, int ncols, int ld_in, int ld_out,
+void yline_real(hipStream_t s, const Batch<T, TI>& io, int nplanes, int ncols, int ld_in, int ld_out,
                 long ps_in, long ps_out, const Twiddle& tin, const Twiddle& tout, LineOp op, double kfac);
 // Pruned half spectra (the test-filtered fields of lagrange_Sdep): only the
 // columns kx < kst are stored, and only the rows y with min(y, n - y) < mc.
 // x r2c (fftn_mpi first half): nrows real rows (length n) -> half-spectrum
 // rows of stride ldc; columns kx < kst are stored (kst < 0: all n/2 + 1).
 template <typename T, typename TI = T>
-void x_r2c(hipStream_t s, const TI* in, cx<T>* out, long nrows, int ld_in, int ldc,
+void x_r2c(hipStream_t s, const Batch<cx<T>, TI>& io, long nrows, int ld_in, int ldc,
            const Twiddle& tw, double scale, int kst = -1);
 // x c2r (ifftn_mpi second half); deriv != 0 applies i*kx (kx Nyquist = 0)
 // first; modes kx >= kst are taken as zero and not read (kst < 0: none).
@@ -209,26 +229,47 @@ void x_c2r(hipStream_t s, const cx<T>* in, T* out, long nrows, int ldc, int ld_o
 // SP_FWD stores and SP_MULINV reads only the rows with min(y, n - y) < mc
 // (the rows outside a filter's support); the other ops take every row.
 template <typename T>
-void yline_spec(hipStream_t s, const cx<T>* in, cx<T>* out, int nplanes, int ncols, long ps,
+void yline_spec(hipStream_t s, const Batch<cx<T>, cx<T>>& io, int nplanes, int ncols, long ps,
                 const Twiddle& tw, SpecOp op, const double* G, int ld = -1, int ldG = -1, int mc = -1);
+// one field
+template <typename T, typename TI = T>
+inline void xline_real(hipStream_t s, const TI* in, T* out, long nrows, int ld_in, int ld_out, const Twiddle& tin,
+                       const Twiddle& tout, LineOp op, double kfac) {
+    xline_real<T, TI>(s, batch1(in, out), nrows, ld_in, ld_out, tin, tout, op, kfac);
+}
+template <typename T, typename TI = T>
+inline void yline_real(hipStream_t s, const TI* in, T* out, int nplanes, int ncols, int ld_in, int ld_out, long ps_in,
+                       long ps_out, const Twiddle& tin, const Twiddle& tout, LineOp op, double kfac) {
+    yline_real<T, TI>(s, batch1(in, out), nplanes, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, op, kfac);
+}
+template <typename T, typename TI = T>
+inline void x_r2c(hipStream_t s, const TI* in, cx<T>* out, long nrows, int ld_in, int ldc, const Twiddle& tw,
+                  double scale, int kst = -1) {
+    x_r2c<T, TI>(s, batch1(in, out), nrows, ld_in, ldc, tw, scale, kst);
+}
+template <typename T>
+inline void yline_spec(hipStream_t s, const cx<T>* in, cx<T>* out, int nplanes, int ncols, long ps, const Twiddle& tw,
+                       SpecOp op, const double* G, int ld = -1, int ldG = -1, int mc = -1) {
+    yline_spec<T>(s, batch1(in, out), nplanes, ncols, ps, tw, op, G, ld, ldG, mc);
+}
 
-// register-radix versions for the production line lengths (k_lines_rg.hip);
+// register-radix versions for compile-time line lengths (k_lines_rg.hip);
 // return false when the
 // line length has no specialisation
 template <typename T, typename TI>
-bool xline_real_ct(hipStream_t s, const TI* in, T* out, long nrows, int ld_in, int ld_out, const Twiddle& tin,
+bool xline_real_ct(hipStream_t s, const Batch<T, TI>& io, long nrows, int ld_in, int ld_out, const Twiddle& tin,
                    const Twiddle& tout, LineOp op, double kfac);
 template <typename T, typename TI>
-bool yline_real_ct(hipStream_t s, const TI* in, T* out, int nplanes, int ncols, int ld_in, int ld_out, long ps_in,
+bool yline_real_ct(hipStream_t s, const Batch<T, TI>& io, int nplanes, int ncols, int ld_in, int ld_out, long ps_in,
                    long ps_out, const Twiddle& tin, const Twiddle& tout, LineOp op, double kfac);
 template <typename T, typename TI>
-bool x_r2c_ct(hipStream_t s, const TI* in, cx<T>* out, long nrows, int ld_in, int ldc, const Twiddle& tw,
+bool x_r2c_ct(hipStream_t s, const Batch<cx<T>, TI>& io, long nrows, int ld_in, int ldc, const Twiddle& tw,
               double scale, int kst);
 template <typename T>
 bool x_c2r_ct(hipStream_t s, const cx<T>* in, T* out, long nrows, int ldc, int ld_out, const Twiddle& tw, int deriv,
               double kfac, int kst);
 template <typename T>
-bool yline_spec_ct(hipStream_t s, const cx<T>* in, cx<T>* out, int nplanes, int ncols, long ps, const Twiddle& tw,
+bool yline_spec_ct(hipStream_t s, const Batch<cx<T>, cx<T>>& io, int nplanes, int ncols, long ps, const Twiddle& tw,
                    SpecOp op, const double* G, int ld, int ldG, int mc);
 // First x passes of a pad / unpad fused with the pointwise function that
 // produces their input (k_lines_rg.hip); false when the line lengths have no
@@ -306,6 +347,8 @@ template <typename W> void lagrange_prep_dev(les_ctx* c, W* buf21);
 template <typename W> void lagrange_contract_dev(les_ctx* c, const W* b2, const W* b4, int init_lm, int init_qn);
 template <typename W, typename TI> void ddz_uv_dev(les_ctx* c, W* d, const TI* f);
 template <typename W, typename TI> void ddz_w_dev(les_ctx* c, W* d, const TI* f);
+template <typename W> void ddz_uvw_dev(les_ctx* c);
+template <typename W> void divstress_combine3_dev(les_ctx* c, W* const a[3], W* const b[3]);
 template <typename W> void divstress_combine_dev(les_ctx* c, W* out, const W* a, const W* b, const W* d, int w_version);
 template <typename W> void vorticity_dev(les_ctx* c, W* v1, W* v2, W* v3);
 template <typename W>

@@ -232,6 +232,14 @@ size_t NP(Run& r) { return r.c->plane; }
 size_t NP2(Run& r) { return r.c->plane2; }
 double* W3(Run& r, int i) { return r.c->work3[i]; }
 
+// batches over linear variables: in -> out, and in -> work3[w0 ..]
+Batch<double, double> triple(Run& r, int a, int b, int c, int oa, int ob, int oc) {
+    return batch3<double, double>(V(r, a), V(r, b), V(r, c), V(r, oa), V(r, ob), V(r, oc));
+}
+Batch<double, double> to_work(Run& r, int a, int b, int c, int w0) {
+    return batch3<double, double>(V(r, a), V(r, b), V(r, c), W3(r, w0), W3(r, w0 + 1), W3(r, w0 + 2));
+}
+
 // lambda_dst(levels l0..l1) += a * unpad(lambda_src(levels l0..l1)) (the
 // transpose of a pad, a = 9/4) or += a * pad(...) (transpose of an unpad, a = 4/9)
 void add_unpad(Run& r, double* dst, double* src, int l0, int l1, double a) {
@@ -241,6 +249,19 @@ void add_unpad(Run& r, double* dst, double* src, int l0, int l1, double a) {
 void add_pad(Run& r, double* dst, double* src, int l0, int l1, double a) {
     if (l1 < l0) return;
     pad_acc_f(r.c, src + (size_t)l0 * NP(r), dst + (size_t)l0 * NP2(r), l1 - l0 + 1, a);
+}
+// the same for three variables in one launch per pass
+void add_unpad3(Run& r, const Batch<double, double>& b, int l0, int l1, double a) {
+    if (l1 < l0) return;
+    Batch<double, double> t = b;
+    for (int f = 0; f < t.nf; ++f) { t.in[f] += (size_t)l0 * NP2(r); t.out[f] += (size_t)l0 * NP(r); }
+    unpad3_f<double>(r.c, t, l1 - l0 + 1, a);
+}
+void add_pad3(Run& r, const Batch<double, double>& b, int l0, int l1, double a) {
+    if (l1 < l0) return;
+    Batch<double, double> t = b;
+    for (int f = 0; f < t.nf; ++f) { t.in[f] += (size_t)l0 * NP(r); t.out[f] += (size_t)l0 * NP2(r); }
+    pad3_f<double, double>(r.c, t, l1 - l0 + 1, a);
 }
 void clear_all(Run& r, int v) { lin_clear(r.c, r.b, V(r, v), (long)lv_size(r.c, v)); }
 
@@ -253,12 +274,8 @@ void s_obk_adj(Run& r) { obk_adj(r.c, r.t, r.b, r.oa); }
 void s_deriv_tl(Run& r) {
     les_ctx* c = r.c;
     const int nl = NL(r);
-    ddx_f<double, double>(c, V(r, L_UX), V(r, L_U), 0, nl);
-    ddy_f<double, double>(c, V(r, L_UY), V(r, L_U), 0, nl);
-    ddx_f<double, double>(c, V(r, L_VX), V(r, L_V), 0, nl);
-    ddy_f<double, double>(c, V(r, L_VY), V(r, L_V), 0, nl);
-    ddx_f<double, double>(c, V(r, L_WX), V(r, L_W), 0, nl);
-    ddy_f<double, double>(c, V(r, L_WY), V(r, L_W), 0, nl);
+    ddx3_f<double, double>(c, triple(r, L_U, L_V, L_W, L_UX, L_VX, L_WX), 0, nl);
+    ddy3_f<double, double>(c, triple(r, L_U, L_V, L_W, L_UY, L_VY, L_WY), 0, nl);
     ddz_uv_tl(c, V(r, L_UZ), V(r, L_U));
     ddz_uv_tl(c, V(r, L_VZ), V(r, L_V));
     ddz_w_tl(c, V(r, L_WZ), V(r, L_W));
@@ -274,9 +291,13 @@ void grad_adj_field(Run& r, int f, int fx, int fy, int fz, int wform) {
     grad_adj(c, V(r, f), W3(r, 0), W3(r, 1), V(r, fz), wform);
 }
 void s_deriv_adj(Run& r) {
-    grad_adj_field(r, L_U, L_UX, L_UY, L_UZ, 0);
-    grad_adj_field(r, L_V, L_VX, L_VY, L_VZ, 0);
-    grad_adj_field(r, L_W, L_WX, L_WY, L_WZ, 1);
+    les_ctx* c = r.c;
+    const int nl = NL(r);
+    ddx3_f<double, double>(c, to_work(r, L_UX, L_VX, L_WX, 0), 0, nl);
+    ddy3_f<double, double>(c, to_work(r, L_UY, L_VY, L_WY, 3), 0, nl);
+    grad_adj(c, V(r, L_U), W3(r, 0), W3(r, 3), V(r, L_UZ), 0);
+    grad_adj(c, V(r, L_V), W3(r, 1), W3(r, 4), V(r, L_VZ), 0);
+    grad_adj(c, V(r, L_W), W3(r, 2), W3(r, 5), V(r, L_WZ), 1);
 }
 
 // 2: filter_data(theta) in place (010_scalars.f90:111-118)
@@ -303,9 +324,10 @@ void s_thpad_tl(Run& r) {
     les_ctx* c = r.c;
     const int nz = NZ(r);
     const size_t np = NP(r), np2 = NP2(r);
-    pad_f<double, double>(c, V(r, L_TX) + np, V(r, L_TB1) + np2, nz - 1);
-    pad_f<double, double>(c, V(r, L_TY) + np, V(r, L_TB2) + np2, nz - 1);
-    pad_f<double, double>(c, V(r, L_TZ) + 2 * np, V(r, L_TB3) + 2 * np2, nz - 1);
+    pad3_f<double, double>(c,
+                           batch3<double, double>(V(r, L_TX) + np, V(r, L_TY) + np, V(r, L_TZ) + 2 * np,
+                                                  V(r, L_TB1) + np2, V(r, L_TB2) + np2, V(r, L_TB3) + 2 * np2),
+                           nz - 1);
 }
 void s_thpad_adj(Run& r) {
     const int nz = NZ(r);
@@ -343,43 +365,31 @@ void s_stress_adj(Run& r) { stress_adj(r.c, r.t, r.b); }
 void s_div_tl(Run& r) {
     les_ctx* c = r.c;
     const int nl = NL(r);
-    double *a = W3(r, 0), *b = W3(r, 1);
-    ddx_f<double, double>(c, a, V(r, L_TXX), 0, nl);
-    ddy_f<double, double>(c, b, V(r, L_TXY), 0, nl);
-    div_tl(c, V(r, L_DVX), a, b, V(r, L_TXZ), 0);
-    ddx_f<double, double>(c, a, V(r, L_TXY), 0, nl);
-    ddy_f<double, double>(c, b, V(r, L_TYY), 0, nl);
-    div_tl(c, V(r, L_DVY), a, b, V(r, L_TYZ), 0);
-    ddx_f<double, double>(c, a, V(r, L_TXZ), 0, nl);
-    ddy_f<double, double>(c, b, V(r, L_TYZ), 0, nl);
-    div_tl(c, V(r, L_DVZ), a, b, V(r, L_TZZ), 1);
+    ddx3_f<double, double>(c, to_work(r, L_TXX, L_TXY, L_TXZ, 0), 0, nl);
+    ddy3_f<double, double>(c, to_work(r, L_TXY, L_TYY, L_TYZ, 3), 0, nl);
+    div_tl(c, V(r, L_DVX), W3(r, 0), W3(r, 3), V(r, L_TXZ), 0);
+    div_tl(c, V(r, L_DVY), W3(r, 1), W3(r, 4), V(r, L_TYZ), 0);
+    div_tl(c, V(r, L_DVZ), W3(r, 2), W3(r, 5), V(r, L_TZZ), 1);
 }
 void s_div_adj(Run& r) {
     les_ctx* c = r.c;
     const int nl = NL(r);
     double* t[6];
     for (int i = 0; i < 6; ++i) t[i] = W3(r, i);
-    ddx_f<double, double>(c, t[0], V(r, L_DVX), 0, nl);
-    ddy_f<double, double>(c, t[1], V(r, L_DVX), 0, nl);
-    ddx_f<double, double>(c, t[2], V(r, L_DVY), 0, nl);
-    ddy_f<double, double>(c, t[3], V(r, L_DVY), 0, nl);
-    ddx_f<double, double>(c, t[4], V(r, L_DVZ), 0, nl);
-    ddy_f<double, double>(c, t[5], V(r, L_DVZ), 0, nl);
+    ddx3_f<double, double>(
+        c, batch3<double, double>(V(r, L_DVX), V(r, L_DVY), V(r, L_DVZ), t[0], t[2], t[4]), 0, nl);
+    ddy3_f<double, double>(
+        c, batch3<double, double>(V(r, L_DVX), V(r, L_DVY), V(r, L_DVZ), t[1], t[3], t[5]), 0, nl);
     div_adj(c, r.b, t);
 }
 
 // 10-14: convec (108_convec.f90)
 void s_cpad_tl(Run& r) {
-    const int nl = NL(r);
-    pad_f<double, double>(r.c, V(r, L_U), V(r, L_UB), nl);
-    pad_f<double, double>(r.c, V(r, L_V), V(r, L_VB), nl);
-    pad_f<double, double>(r.c, V(r, L_W), V(r, L_WB), nl);
+    pad3_f<double, double>(r.c, triple(r, L_U, L_V, L_W, L_UB, L_VB, L_WB), NL(r));
 }
 void s_cpad_adj(Run& r) {
     const int nz = NZ(r);
-    add_unpad(r, V(r, L_U), V(r, L_UB), 1, nz - 1, 9.0 / 4.0);
-    add_unpad(r, V(r, L_V), V(r, L_VB), 1, nz - 1, 9.0 / 4.0);
-    add_unpad(r, V(r, L_W), V(r, L_WB), 1, nz - 1, 9.0 / 4.0);
+    add_unpad3(r, triple(r, L_UB, L_VB, L_WB, L_U, L_V, L_W), 1, nz - 1, 9.0 / 4.0);
     // no clearing: the scalar advection's adjoint writes levels 1..nz-1 first
 }
 void s_vort_tl(Run& r) { vort_tl(r.c, r.b); }
@@ -387,26 +397,30 @@ void s_vort_adj(Run& r) { vort_adj(r.c, r.b); }
 void s_vpad_tl(Run& r) {
     const int nz = NZ(r);
     const size_t np = NP(r), np2 = NP2(r);
-    for (int m = 0; m < 3; ++m) pad_f<double, double>(r.c, V(r, L_O1 + m) + np, V(r, L_OB1 + m) + np2, nz);
+    pad3_f<double, double>(r.c,
+                           batch3<double, double>(V(r, L_O1) + np, V(r, L_O1 + 1) + np, V(r, L_O1 + 2) + np,
+                                                  V(r, L_OB1) + np2, V(r, L_OB1 + 1) + np2, V(r, L_OB1 + 2) + np2),
+                           nz);
 }
 void s_vpad_adj(Run& r) {
     const int nz = NZ(r);
-    for (int m = 0; m < 3; ++m) {
-        add_unpad(r, V(r, L_O1 + m), V(r, L_OB1 + m), 1, nz, 9.0 / 4.0);  // the cross product writes these
-    }
+    // the cross product writes these
+    add_unpad3(r, triple(r, L_OB1, L_OB1 + 1, L_OB1 + 2, L_O1, L_O1 + 1, L_O1 + 2), 1, nz, 9.0 / 4.0);
 }
 void s_cross_tl(Run& r) { cross_tl(r.c, r.t, r.b); }
 void s_cross_adj(Run& r) { cross_adj(r.c, r.t, r.b); }
 void s_cunpad_tl(Run& r) {
     const int nz = NZ(r);
     const size_t np = NP(r), np2 = NP2(r);
-    for (int m = 0; m < 3; ++m) unpad_f<double>(r.c, V(r, L_CB1 + m) + np2, V(r, L_CX + m) + np, nz - 1);
+    unpad3_f<double>(r.c,
+                     batch3<double, double>(V(r, L_CB1) + np2, V(r, L_CB1 + 1) + np2, V(r, L_CB1 + 2) + np2,
+                                            V(r, L_CX) + np, V(r, L_CX + 1) + np, V(r, L_CX + 2) + np),
+                     nz - 1);
 }
 void s_cunpad_adj(Run& r) {
     const int nz = NZ(r);
-    for (int m = 0; m < 3; ++m) {
-        add_pad(r, V(r, L_CB1 + m), V(r, L_CX + m), 1, nz - 1, 4.0 / 9.0);  // rhs writes lambda_C
-    }
+    // rhs writes lambda_C
+    add_pad3(r, triple(r, L_CX, L_CX + 1, L_CX + 2, L_CB1, L_CB1 + 1, L_CB1 + 2), 1, nz - 1, 4.0 / 9.0);
 }
 
 // 15-20: scalar RHS, calc_beta, step_scalar (010_scalars.f90:466-671)
@@ -462,7 +476,7 @@ void s_gradp_adj(Run& r) {
 void s_proj_tl(Run& r) { project_tl(r.c, r.b, r.sf); }
 void s_proj_adj(Run& r) { project_adj(r.c, r.b, r.sf); }
 void s_filt(Run& r) {
-    for (int m = 0; m < 3; ++m) filter_f<double>(r.c, V(r, L_U + m), 0, NL(r));
+    filter3_f(r.c, V(r, L_U), V(r, L_U + 1), V(r, L_U + 2), NL(r));
 }
 
 struct Reg {

@@ -70,6 +70,47 @@ inline void unpad_acc_f(les_ctx* c, const double* src, double* dst, int nlev, do
     yline_real<double>(c->stream, tmp, dst, nlev, c->nx, c->nx, c->nx, (long)c->ny2 * c->nx, (long)c->plane,
                        c->tw_y2, c->tw_y, OP_UNPAD, acc);
 }
+// the same on three fields in one launch per pass
+template <typename W, typename TI>
+inline void ddx3_f(les_ctx* c, const Batch<W, TI>& io, int lev0, int nlev) {
+    Batch<W, TI> b = io;
+    for (int f = 0; f < b.nf; ++f) { b.in[f] += (size_t)lev0 * c->plane; b.out[f] += (size_t)lev0 * c->plane; }
+    xline_real<W, TI>(c->stream, b, (long)nlev * c->ny, c->nx, c->nx, c->tw_x, c->tw_x, OP_DERIV, kfx(c));
+}
+template <typename W, typename TI>
+inline void ddy3_f(les_ctx* c, const Batch<W, TI>& io, int lev0, int nlev) {
+    Batch<W, TI> b = io;
+    for (int f = 0; f < b.nf; ++f) { b.in[f] += (size_t)lev0 * c->plane; b.out[f] += (size_t)lev0 * c->plane; }
+    yline_real<W, TI>(c->stream, b, nlev, c->nx, c->nx, c->nx, (long)c->plane, (long)c->plane, c->tw_y, c->tw_y,
+                      OP_DERIV, kfy(c));
+}
+inline void filter3_f(les_ctx* c, double* u, double* v, double* w, int nlev) {
+    const Batch<double, double> b = batch3<double, double>(u, v, w, u, v, w);
+    xline_real<double>(c->stream, b, (long)nlev * c->ny, c->nx, c->nx, c->tw_x, c->tw_x, OP_NYQ, 0.0);
+    yline_real<double>(c->stream, b, nlev, c->nx, c->nx, c->nx, (long)c->plane, (long)c->plane, c->tw_y, c->tw_y,
+                       OP_NYQ, 0.0);
+}
+// acc as in pad_acc_f (0: written)
+template <typename W, typename TI>
+inline void pad3_f(les_ctx* c, const Batch<W, TI>& io, int nlev, double acc = 0.0) {
+    const size_t S = (size_t)nlev * c->ny * c->nx2;   // work3[6] holds three
+    W* t = scr<W>(c->work3[6]);
+    const Batch<W, TI> bx{io.nf, {io.in[0], io.in[1], io.in[2]}, {t, t + S, t + 2 * S}};
+    const Batch<W, W> by{io.nf, {t, t + S, t + 2 * S}, {io.out[0], io.out[1], io.out[2]}};
+    xline_real<W, TI>(c->stream, bx, (long)nlev * c->ny, c->nx, c->nx2, c->tw_x, c->tw_x2, OP_PAD, 0.0);
+    yline_real<W>(c->stream, by, nlev, c->nx2, c->nx2, c->nx2, (long)c->ny * c->nx2, (long)c->plane2, c->tw_y,
+                  c->tw_y2, OP_PAD, acc);
+}
+template <typename W>
+inline void unpad3_f(les_ctx* c, const Batch<W, W>& io, int nlev, double acc = 0.0) {
+    const size_t S = (size_t)nlev * c->ny2 * c->nx;
+    W* t = scr<W>(c->work3[6]);
+    const Batch<W, W> bx{io.nf, {io.in[0], io.in[1], io.in[2]}, {t, t + S, t + 2 * S}};
+    const Batch<W, W> by{io.nf, {t, t + S, t + 2 * S}, {io.out[0], io.out[1], io.out[2]}};
+    xline_real<W>(c->stream, bx, (long)nlev * c->ny2, c->nx2, c->nx, c->tw_x2, c->tw_x, OP_UNPAD, 0.0);
+    yline_real<W>(c->stream, by, nlev, c->nx, c->nx, c->nx, (long)c->ny2 * c->nx, (long)c->plane, c->tw_y2, c->tw_y,
+                  OP_UNPAD, acc);
+}
 // test_filter of nplanes consecutive planes in place
 template <typename T>
 inline void test_filter_f(les_ctx* c, T* p, int nplanes, const double* G) {

@@ -304,10 +304,18 @@ constexpr int rg_threads() {
     return round64(rg_lines<T, NIN, NOUT, YM>() * cmax(rg_maxbf(NIN), rg_maxbf(NOUT)));
 }
 
+// field f of a batch (f is uniform: a scalar select)
+template <typename P>
+__device__ __forceinline__ P pick(P const (&p)[BATCH], unsigned f) {
+    return f == 0 ? p[0] : (f == 1 ? p[1] : p[2]);
+}
+
 template <typename T, typename TI, int NIN, int NOUT, int OP>
 __global__ __launch_bounds__((rg_threads<T, NIN, NOUT, false>())) void kr_xline(
-    const TI* __restrict__ in, T* __restrict__ out, long nrows, int ld_in, int ld_out,
+    Batch<T, TI> io, long nrows, int ld_in, int ld_out,
     const cx<T>* __restrict__ twin_g, const cx<T>* __restrict__ twout_g, T kfac) {
+    const TI* __restrict__ in = pick(io.in, blockIdx.y);
+    T* __restrict__ out = pick(io.out, blockIdx.y);
     constexpr int NL = rg_lines<T, NIN, NOUT, false>();
     constexpr int NTH = rg_threads<T, NIN, NOUT, false>();
     constexpr int LS = rg_ls(cmax(NIN, NOUT));
@@ -364,8 +372,10 @@ __global__ __launch_bounds__((rg_threads<T, NIN, NOUT, false>())) void kr_xline(
 
 template <typename T, typename TI, int NIN, int NOUT, int OP>
 __global__ __launch_bounds__((rg_threads<T, NIN, NOUT, true>())) void kr_yline(
-    const TI* __restrict__ in, T* __restrict__ out, int ncols, int ld_in, int ld_out, long ps_in, long ps_out,
+    Batch<T, TI> io, int ncols, int ld_in, int ld_out, long ps_in, long ps_out,
     const cx<T>* __restrict__ twin_g, const cx<T>* __restrict__ twout_g, T kfac) {
+    const TI* __restrict__ in = pick(io.in, blockIdx.z);
+    T* __restrict__ out = pick(io.out, blockIdx.z);
     constexpr int NL = rg_lines<T, NIN, NOUT, true>();
     constexpr int NTH = rg_threads<T, NIN, NOUT, true>();
     constexpr int LS = rg_ls(cmax(NIN, NOUT));
@@ -475,10 +485,11 @@ __device__ __forceinline__ void r2c_body(const LD& ld, const ROW& row, int LH, c
 // x r2c of fftn_mpi (FFTW r2c: k = 0..N/2; the x Nyquist is zeroed as in
 // fftn_mpi), two real rows per complex line, split by Hermitian symmetry.
 template <typename T, typename TI, int N>
-__global__ __launch_bounds__((rg_threads<T, N, N, false>())) void kr_x_r2c(const TI* __restrict__ in,
-                                                                         cx<T>* __restrict__ out, long nrows,
+__global__ __launch_bounds__((rg_threads<T, N, N, false>())) void kr_x_r2c(Batch<cx<T>, TI> io, long nrows,
                                                                          int ld_in, int ldc, int kst,
                                                                          const cx<T>* __restrict__ tw_g, T scale) {
+    const TI* __restrict__ in = pick(io.in, blockIdx.y);
+    cx<T>* __restrict__ out = pick(io.out, blockIdx.y);
     constexpr int NL = rg_lines<T, N, N, false>();
     constexpr int NTH = rg_threads<T, N, N, false>();
     constexpr int LS = rg_ls(N);
@@ -551,11 +562,12 @@ __global__ __launch_bounds__((rg_threads<T, N, N, false>())) void kr_x_c2r(const
 // rows per plane); SP_FWD stores and SP_MULINV reads only the rows with
 // min(p, N - p) < mc
 template <typename T, int N, int OP>
-__global__ __launch_bounds__((rg_threads<T, N, N, true>())) void kr_yspec(const cx<T>* __restrict__ in,
-                                                                        cx<T>* __restrict__ out, int ncols, int ld,
+__global__ __launch_bounds__((rg_threads<T, N, N, true>())) void kr_yspec(Batch<cx<T>, cx<T>> io, int ncols, int ld,
                                                                         int ldG, int mc, long ps,
                                                                         const cx<T>* __restrict__ tw_g,
                                                                         const double* __restrict__ G) {
+    const cx<T>* __restrict__ in = pick(io.in, blockIdx.z);
+    cx<T>* __restrict__ out = pick(io.out, blockIdx.z);
     // one complex column per line: 8 (FP64) / 16 (FP32) columns = 128 bytes
     constexpr int NL = rg_lines<T, N, N, true>();
     constexpr int NTH = rg_threads<T, N, N, true>();
@@ -909,15 +921,15 @@ inline const cx<T>* twp(const Twiddle& t) {
 // x and y return false for an op the input types have no kernel for.
 template <typename T, typename TI>
 struct RgIo {
-    bool (*x)(hipStream_t, LineOp, const TI*, T*, long, int, int, const Twiddle&, const Twiddle&, double);
-    bool (*y)(hipStream_t, LineOp, const TI*, T*, int, int, int, int, long, long, const Twiddle&, const Twiddle&,
+    bool (*x)(hipStream_t, LineOp, const Batch<T, TI>&, long, int, int, const Twiddle&, const Twiddle&, double);
+    bool (*y)(hipStream_t, LineOp, const Batch<T, TI>&, int, int, int, int, long, long, const Twiddle&, const Twiddle&,
               double);
-    void (*r2c)(hipStream_t, const TI*, cx<T>*, long, int, int, const Twiddle&, double, int);
+    void (*r2c)(hipStream_t, const Batch<cx<T>, TI>&, long, int, int, const Twiddle&, double, int);
 };
 template <typename T>
 struct RgOps {
     void (*c2r)(hipStream_t, const cx<T>*, T*, long, int, int, const Twiddle&, int, double, int);
-    void (*spec)(hipStream_t, SpecOp, const cx<T>*, cx<T>*, int, int, long, const Twiddle&, const double*, int, int,
+    void (*spec)(hipStream_t, SpecOp, const Batch<cx<T>, cx<T>>&, int, int, long, const Twiddle&, const double*, int, int,
                  int);
     void (*cross)(hipStream_t, const ConvIn<T>&, int, T*, T*, T*, int, int, const Twiddle&, const Twiddle&);
     void (*vort)(hipStream_t, const VortIn<T>&, T*, T*, T*, int, int, const Twiddle&, const Twiddle&);
@@ -934,53 +946,53 @@ struct RgTable {
 };
 
 template <typename T, typename TI, int NIN, int NOUT, int OP>
-void launch_x(hipStream_t s, const TI* in, T* out, long nrows, int ld_in, int ld_out, const Twiddle& tin,
+void launch_x(hipStream_t s, const Batch<T, TI>& io, long nrows, int ld_in, int ld_out, const Twiddle& tin,
               const Twiddle& tout, double kfac) {
     constexpr int NL = rg_lines<T, NIN, NOUT, false>();
     constexpr int NTH = rg_threads<T, NIN, NOUT, false>();
     const long nb = (nrows + 2 * NL - 1) / (2 * NL);
-    hipLaunchKernelGGL((kr_xline<T, TI, NIN, NOUT, OP>), dim3((unsigned)nb), dim3(NTH), 0, s, in, out, nrows, ld_in,
+    hipLaunchKernelGGL((kr_xline<T, TI, NIN, NOUT, OP>), dim3((unsigned)nb, io.nf), dim3(NTH), 0, s, io, nrows, ld_in,
                        ld_out, twp<T>(tin), twp<T>(tout), (T)kfac);
 }
 
 template <typename T, typename TI, int NIN, int NOUT, int OP>
-void launch_y(hipStream_t s, const TI* in, T* out, int nplanes, int ncols, int ld_in, int ld_out, long ps_in,
+void launch_y(hipStream_t s, const Batch<T, TI>& io, int nplanes, int ncols, int ld_in, int ld_out, long ps_in,
               long ps_out, const Twiddle& tin, const Twiddle& tout, double kfac) {
     constexpr int NL = rg_lines<T, NIN, NOUT, true>();
     constexpr int NTH = rg_threads<T, NIN, NOUT, true>();
     const int nbx = (ncols + 2 * NL - 1) / (2 * NL);
-    hipLaunchKernelGGL((kr_yline<T, TI, NIN, NOUT, OP>), dim3(nbx, nplanes), dim3(NTH), 0, s, in, out, ncols, ld_in,
+    hipLaunchKernelGGL((kr_yline<T, TI, NIN, NOUT, OP>), dim3(nbx, nplanes, io.nf), dim3(NTH), 0, s, io, ncols, ld_in,
                        ld_out, ps_in, ps_out, twp<T>(tin), twp<T>(tout), (T)kfac);
 }
 
 template <typename T, typename TI, int N>
 struct RgIoOf {
-    static bool x(hipStream_t s, LineOp op, const TI* in, T* out, long nrows, int ld_in, int ld_out,
+    static bool x(hipStream_t s, LineOp op, const Batch<T, TI>& io, long nrows, int ld_in, int ld_out,
                   const Twiddle& tin, const Twiddle& tout, double kfac) {
         constexpr int M = 3 * N / 2;
-        if (op == OP_DERIV) launch_x<T, TI, N, N, OP_DERIV>(s, in, out, nrows, ld_in, ld_out, tin, tout, kfac);
-        else if (op == OP_PAD) launch_x<T, TI, N, M, OP_PAD>(s, in, out, nrows, ld_in, ld_out, tin, tout, kfac);
+        if (op == OP_DERIV) launch_x<T, TI, N, N, OP_DERIV>(s, io, nrows, ld_in, ld_out, tin, tout, kfac);
+        else if (op == OP_PAD) launch_x<T, TI, N, M, OP_PAD>(s, io, nrows, ld_in, ld_out, tin, tout, kfac);
         else if constexpr (sizeof(T) != sizeof(TI)) return false;
-        else if (op == OP_NYQ) launch_x<T, TI, N, N, OP_NYQ>(s, in, out, nrows, ld_in, ld_out, tin, tout, kfac);
-        else launch_x<T, TI, M, N, OP_UNPAD>(s, in, out, nrows, ld_in, ld_out, tin, tout, kfac);
+        else if (op == OP_NYQ) launch_x<T, TI, N, N, OP_NYQ>(s, io, nrows, ld_in, ld_out, tin, tout, kfac);
+        else launch_x<T, TI, M, N, OP_UNPAD>(s, io, nrows, ld_in, ld_out, tin, tout, kfac);
         return true;
     }
-    static bool y(hipStream_t s, LineOp op, const TI* in, T* out, int np, int ncols, int ld_in, int ld_out, long ps_in,
+    static bool y(hipStream_t s, LineOp op, const Batch<T, TI>& io, int np, int ncols, int ld_in, int ld_out, long ps_in,
                   long ps_out, const Twiddle& tin, const Twiddle& tout, double kfac) {
         constexpr int M = 3 * N / 2;
-        if (op == OP_DERIV) launch_y<T, TI, N, N, OP_DERIV>(s, in, out, np, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, kfac);
-        else if (op == OP_PAD) launch_y<T, TI, N, M, OP_PAD>(s, in, out, np, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, kfac);
+        if (op == OP_DERIV) launch_y<T, TI, N, N, OP_DERIV>(s, io, np, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, kfac);
+        else if (op == OP_PAD) launch_y<T, TI, N, M, OP_PAD>(s, io, np, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, kfac);
         else if constexpr (sizeof(T) != sizeof(TI)) return false;
-        else if (op == OP_NYQ) launch_y<T, TI, N, N, OP_NYQ>(s, in, out, np, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, kfac);
-        else launch_y<T, TI, M, N, OP_UNPAD>(s, in, out, np, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, kfac);
+        else if (op == OP_NYQ) launch_y<T, TI, N, N, OP_NYQ>(s, io, np, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, kfac);
+        else launch_y<T, TI, M, N, OP_UNPAD>(s, io, np, ncols, ld_in, ld_out, ps_in, ps_out, tin, tout, kfac);
         return true;
     }
-    static void r2c(hipStream_t s, const TI* in, cx<T>* out, long nrows, int ld_in, int ldc, const Twiddle& tw,
+    static void r2c(hipStream_t s, const Batch<cx<T>, TI>& io, long nrows, int ld_in, int ldc, const Twiddle& tw,
                     double scale, int kst) {
         constexpr int NL = rg_lines<T, N, N, false>();
         constexpr int NTH = rg_threads<T, N, N, false>();
         const long nb = (nrows + 2 * NL - 1) / (2 * NL);
-        hipLaunchKernelGGL((kr_x_r2c<T, TI, N>), dim3((unsigned)nb), dim3(NTH), 0, s, in, out, nrows, ld_in, ldc, kst,
+        hipLaunchKernelGGL((kr_x_r2c<T, TI, N>), dim3((unsigned)nb, io.nf), dim3(NTH), 0, s, io, nrows, ld_in, ldc, kst,
                            twp<T>(tw), (T)scale);
     }
     static constexpr RgIo<T, TI> table() { return {x, y, r2c}; }
@@ -1003,21 +1015,21 @@ struct RgOpsOf {
         else c2r_d<0>(s, in, out, nrows, ldc, ld_out, tw, kfac, kst);
     }
     template <int OP>
-    static void spec_o(hipStream_t s, const cx<T>* in, cx<T>* out, int nplanes, int ncols, long ps, const Twiddle& tw,
+    static void spec_o(hipStream_t s, const Batch<cx<T>, cx<T>>& io, int nplanes, int ncols, long ps, const Twiddle& tw,
                        const double* G, int ld, int ldG, int mc) {
         constexpr int NL = rg_lines<T, N, N, true>();
         constexpr int NTH = rg_threads<T, N, N, true>();
         const int nbx = (ncols + NL - 1) / NL;
-        hipLaunchKernelGGL((kr_yspec<T, N, OP>), dim3(nbx, nplanes), dim3(NTH), 0, s, in, out, ncols, ld, ldG, mc, ps,
+        hipLaunchKernelGGL((kr_yspec<T, N, OP>), dim3(nbx, nplanes, io.nf), dim3(NTH), 0, s, io, ncols, ld, ldG, mc, ps,
                            twp<T>(tw), G);
     }
-    static void spec(hipStream_t s, SpecOp op, const cx<T>* in, cx<T>* out, int np, int ncols, long ps,
+    static void spec(hipStream_t s, SpecOp op, const Batch<cx<T>, cx<T>>& io, int np, int ncols, long ps,
                      const Twiddle& tw, const double* G, int ld, int ldG, int mc) {
         switch (op) {
-            case SP_FWD: spec_o<SP_FWD>(s, in, out, np, ncols, ps, tw, G, ld, ldG, mc); break;
-            case SP_INV: spec_o<SP_INV>(s, in, out, np, ncols, ps, tw, G, ld, ldG, mc); break;
-            case SP_FILT: spec_o<SP_FILT>(s, in, out, np, ncols, ps, tw, G, ld, ldG, mc); break;
-            default: spec_o<SP_MULINV>(s, in, out, np, ncols, ps, tw, G, ld, ldG, mc); break;
+            case SP_FWD: spec_o<SP_FWD>(s, io, np, ncols, ps, tw, G, ld, ldG, mc); break;
+            case SP_INV: spec_o<SP_INV>(s, io, np, ncols, ps, tw, G, ld, ldG, mc); break;
+            case SP_FILT: spec_o<SP_FILT>(s, io, np, ncols, ps, tw, G, ld, ldG, mc); break;
+            default: spec_o<SP_MULINV>(s, io, np, ncols, ps, tw, G, ld, ldG, mc); break;
         }
     }
     template <int NIN, int NOUT, int OP, int NC, typename IN>
