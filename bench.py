@@ -294,13 +294,13 @@ _POINT_FAMILIES = [
     (("k_rhs_ab2",), "rhs_ab2"),
     (("k_gradp_project", "k_project_bc"), "gradp_project"),
     (("k_strain_stress", "k_strain<", "k_stress<"), "sgs_stress"),
-    (("k_scalar_flux", "k_scalar_accum", "k_ddz_w_accum"), "scalar_flux"),
-    (("k_ddz_uv", "k_ddz_w<"), "ddz"),
+    (("k_scalar_flux", "k_scalar_accum", "k_scalar_rhs_step"), "scalar_flux"),
+    (("k_ddz_uv", "k_ddz_w<", "k_theta_grad"), "ddz"),
     (("k_divstress",), "divstress"),
     (("k_max3_lag", "k_max3_part", "k_max3_final"), "cfl_max"),
     (("k_press_prep", "k_dpdz", "k_hz_part", "k_hz_fold"), "press_prep"),
     (("k_lag_prep", "k_interpolag", "k_lag_contract<", "k_lag_acc"), "lagrange_point"),
-    (("k_theta_prep", "k_step_scalar", "k_calc_beta", "k_scalar_top"), "theta_point"),
+    (("k_step_scalar", "k_calc_beta", "k_scalar_top"), "theta_point"),
     (("k_tdma",), "tdma"),
     (("kr_lag_contract",), "lag_contract_x"),
     (("kr_x_r2c", "k_x_r2c"), "x_r2c"),

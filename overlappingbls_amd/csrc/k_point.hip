@@ -1042,22 +1042,35 @@ void cross_product_dev(les_ctx* c, const W* b1, const W* b2, const W* b3, W* cxb
 }
 
 // ---- scalar transport, 010_scalars.f90:111-671 ----------------------------------
+// dTdz (ddz_uv, with the prescribed gradient at the top, :137-140) in one pass.
+// The RHS history (:130-135) is a buffer exchange before this kernel: rhsf
+// holds the last step's RHS and rhs is rewritten on levels 1..nz-1 later in
+// the step, so only the ghost levels 0 and nz are carried over here (a whole
+// copy took 168 us at 256^3).
 template <typename W>
-__global__ void k_theta_prep(W* dTdz, double* rhsf, const double* __restrict__ rhs, KP p, double top) {
+__global__ void k_theta_grad(W* dTdz, const double* __restrict__ th, double* rhs, const double* __restrict__ rhsf,
+                             KP p, double top) {
     const long n = p.plane * (p.nz + 1);
+    const double cst = 1.0 / p.dz;
     GRID_LOOP(i, n) {
-        rhsf[i] = rhs[i];
-        if (i >= p.plane * p.nz) dTdz[i] = top;
+        const int k = (int)(i / p.plane);
+        if (k == 0 || k == p.nz) {
+            dTdz[i] = (k == 0) ? BOGUS : top;
+            rhs[i] = rhsf[i];
+        } else if (k >= 2) {
+            dTdz[i] = cst * (th[i] - th[i - p.plane]);
+        }
     }
 }
 
 template <typename W>
-void theta_prep_dev(les_ctx* c) {
-    FamScope fs(c->stream, FAM_THETA_POINT, (2.0 * sizeof(W) + 16.0) * (double)c->plane * (double)c->nlev);
+void theta_grad_dev(les_ctx* c) {
+    FamScope fs(c->stream, FAM_DDZ, (sizeof(W) + 8.0) * (double)c->plane * (double)c->nlev);
     KP p = kp(c);
     const les_params& P = c->prm;
-    hipLaunchKernelGGL(k_theta_prep<W>, grid_for(p.plane * (p.nz + 1)), dim3(256), 0, c->stream, WF<W>(c, LES_F_DTDZ),
-                       c->f3[LES_F_RHST_F], (const double*)c->f3[LES_F_RHST], p, P.dTdz_top / P.T_scale * P.z_i);
+    hipLaunchKernelGGL(k_theta_grad<W>, grid_for(p.plane * (p.nz + 1)), dim3(256), 0, c->stream, WF<W>(c, LES_F_DTDZ),
+                       (const double*)c->f3[LES_F_THETA], c->f3[LES_F_RHST], (const double*)c->f3[LES_F_RHST_F], p,
+                       P.dTdz_top / P.T_scale * P.z_i);
 }
 
 // dealiased advection on the 3/2 grid, levels 1..nz-1 (:466-484)
@@ -1086,7 +1099,6 @@ void scalar_adv_dev(les_ctx* c, const W* dsx, const W* dsy, const W* dsz, W* rm)
                        (const double*)c->ust, (const double*)c->vst, rm, p);
 }
 
-// SGS flux components: comp 0 x (:513-541), 1 y (:552-569), 2 z (:578-594)
 // Surface flux of scalar_RHS_calc (010_scalars.f90:359-394): lbc = 1 the
 // prescribed wt_s (surf_flux); lbc = 0 the bulk Monin-Obukhov flux from the
 // surface temperature T_s and the filtered theta of level 1, with ustar_avg
@@ -1129,11 +1141,8 @@ __global__ void k_scalar_flux(W* temp, double* sgs_t3, const W* __restrict__ Nu,
 }
 
 template <typename W>
-void scalar_flux_dev(les_ctx* c, W* temp, int comp) {
-    FamScope fs(c->stream, FAM_SCALAR_FLUX, (3.0 * sizeof(W) + (comp == 2 ? 8.0 : 0.0)) * (double)c->plane * (double)c->nlev);
-    KP p = kp(c);
+static SurfFlux surf_flux_args(les_ctx* c) {
     const les_params& P = c->prm;
-    const W* ds = WF<W>(c, comp == 0 ? LES_F_DTDX : comp == 1 ? LES_F_DTDY : LES_F_DTDZ);
     SurfFlux sf;
     sf.bulk = (P.lbc == 0);
     sf.surf_flux = P.wt_s / P.T_scale / P.u_scale;
@@ -1142,8 +1151,111 @@ void scalar_flux_dev(les_ctx* c, W* temp, int comp) {
     sf.th1 = c->f3[LES_F_THETA] + c->plane;
     sf.ustar = c->ustar;
     sf.psi_h = c->psi_h;
+    return sf;
+}
+
+template <typename W>
+void scalar_flux_dev(les_ctx* c, W* temp, int comp) {
+    FamScope fs(c->stream, FAM_SCALAR_FLUX, (3.0 * sizeof(W) + (comp == 2 ? 8.0 : 0.0)) * (double)c->plane * (double)c->nlev);
+    KP p = kp(c);
+    const W* ds = WF<W>(c, comp == 0 ? LES_F_DTDX : comp == 1 ? LES_F_DTDY : LES_F_DTDZ);
     hipLaunchKernelGGL(k_scalar_flux<W>, grid_for(p.plane * (p.nz + 1)), dim3(256), 0, c->stream, temp,
-                       c->f3[LES_F_SGS_T3], (const W*)WF<W>(c, LES_F_NU_T), ds, p, comp, 1.0 / P.Pr, sf);
+                       c->f3[LES_F_SGS_T3], (const W*)WF<W>(c, LES_F_NU_T), ds, p, comp, 1.0 / c->prm.Pr,
+                       surf_flux_args<W>(c));
+}
+
+// Both horizontal flux components in one pass over Nu_t (comp 0 and 1 of
+// k_scalar_flux, the same values)
+template <typename W>
+__global__ void k_scalar_flux_xy(W* fx, W* fy, const W* __restrict__ Nu, const W* __restrict__ dx,
+                                 const W* __restrict__ dy, KP p, double iPr) {
+    const long n = p.plane * (p.nz + 1);
+    GRID_LOOP(i, n) {
+        const int k = (int)(i / p.plane);
+        double tx = 0.0, ty = 0.0;
+        if (k >= 1 && k <= p.nz - 1) {
+            if (k == 1) {
+                tx = iPr * Nu[i] * dx[i];
+                ty = iPr * Nu[i] * dy[i];
+            } else if (k == p.nz - 1) {
+                tx = iPr * Nu[i + p.plane] * dx[i];
+                ty = iPr * Nu[i + p.plane] * dy[i];
+            } else {
+                const double c = iPr * 0.5 * ((double)Nu[i] + (double)Nu[i + p.plane]);
+                tx = c * dx[i];
+                ty = c * dy[i];
+            }
+        }
+        fx[i] = tx;
+        fy[i] = ty;
+    }
+}
+
+template <typename W>
+void scalar_flux_xy_dev(les_ctx* c, W* fx, W* fy) {
+    FamScope fs(c->stream, FAM_SCALAR_FLUX, 5.0 * sizeof(W) * (double)c->plane * (double)c->nlev);
+    KP p = kp(c);
+    hipLaunchKernelGGL(k_scalar_flux_xy<W>, grid_for(p.plane * (p.nz + 1)), dim3(256), 0, c->stream, fx, fy,
+                       (const W*)WF<W>(c, LES_F_NU_T), (const W*)WF<W>(c, LES_F_DTDX), (const W*)WF<W>(c, LES_F_DTDY),
+                       p, 1.0 / c->prm.Pr);
+}
+
+// The rest of theta's step in one pass: the vertical flux formed from Nu_t and
+// dTdz and differenced in registers, RHS = -adv + dx + dy + dz (summed in
+// that order, each term rounded to W as the separate kernels store it), the
+// AB2 update of step_scalar (:624-671) and the boundary rows.  Ten field
+// passes instead of the seventeen of k_scalar_flux (z), k_scalar_accum (twice),
+// ddz_w with its accumulation, and k_step_scalar; bound by HBM.  With
+// k_scalar_flux_xy and k_theta_grad a 10-step window at 256^3 takes 109.6
+// against 115.5 ms (mixed 79.6 against 83.2 ms).
+//  euler: RHS_f <- RHS first; rows: theta's rows 0 and nz <- BOGUS (project's),
+//  else row nz from step_scalar's top rule.
+template <typename W>
+__global__ void k_scalar_rhs_step(double* th, double* rhs, double* rhsf, double* sgs_t3, const W* __restrict__ adv,
+                                  const W* __restrict__ dx, const W* __restrict__ dy, const W* __restrict__ Nu,
+                                  const W* __restrict__ dTdz, KP p, double iPr, SurfFlux sf, int euler, int rows,
+                                  int above1, double topgrad) {
+    const long n = p.plane * (p.nz - 1);   // levels 1..nz-1
+    const double cst = 1.0 / p.dz;
+    GRID_LOOP(t, n) {
+        const long i = p.plane + t, j = i + p.plane;
+        const int k = (int)(i / p.plane);
+        double f0, f1;
+        if (k == 1) {
+            const double fl = surf_flux_at(sf, t);
+            f0 = -1.0 * fl;
+            sgs_t3[i] = fl;
+        } else {
+            f0 = iPr * Nu[i] * dTdz[i];
+            sgs_t3[i] = -1.0 * f0;
+        }
+        f1 = iPr * Nu[j] * dTdz[j];
+        if (k == p.nz - 1) sgs_t3[j] = -1.0 * f1;
+        const W dz = (W)(cst * ((double)(W)f1 - (double)(W)f0));
+        double r = -1.0 * (double)adv[i] + dx[i];
+        r = r + dy[i];
+        r = r + (double)dz;
+        rhs[i] = r;
+        double rf = r;
+        if (euler) rhsf[i] = r;
+        else rf = rhsf[i];
+        const double v = th[i] + p.dt * (1.5 * r - 0.5 * rf);
+        th[i] = v;
+        if (k == p.nz - 1) th[j] = rows ? BOGUS : (above1 ? v + topgrad : v);
+        if (k == 1 && rows) th[t] = BOGUS;
+    }
+}
+
+template <typename W>
+void scalar_rhs_step_dev(les_ctx* c, const W* adv, const W* dx, const W* dy, bool euler, bool rows) {
+    FamScope fs(c->stream, FAM_SCALAR_FLUX, (5.0 * sizeof(W) + 40.0) * (double)c->plane * (double)c->nlev);
+    KP p = kp(c);
+    const les_params& P = c->prm;
+    hipLaunchKernelGGL(k_scalar_rhs_step<W>, grid_for(p.plane * (p.nz - 1)), dim3(256), 0, c->stream,
+                       c->f3[LES_F_THETA], c->f3[LES_F_RHST], c->f3[LES_F_RHST_F], c->f3[LES_F_SGS_T3], adv, dx, dy,
+                       (const W*)WF<W>(c, LES_F_NU_T), (const W*)WF<W>(c, LES_F_DTDZ), p, 1.0 / P.Pr,
+                       surf_flux_args<W>(c), (int)euler, (int)rows, (int)(P.lz_npz > 1.0),
+                       P.dTdz_top / P.T_scale * P.z_i * c->dz);
 }
 
 // adv != null: RHS = -adv + d (first flux, adv = the advection term), else
@@ -1155,27 +1267,6 @@ __global__ void k_scalar_accum(double* rhs, const W* __restrict__ d, const W* __
         const long i = p.plane + t;
         rhs[i] = adv ? (-1.0 * (double)adv[i] + d[i]) : (rhs[i] + d[i]);
     }
-}
-
-// ddz_w of the vertical flux (rounded to W as k_ddz_w stores it) added to the
-// RHS at once (k_scalar_accum without adv), levels 1..nz-1
-template <typename W>
-__global__ void k_ddz_w_accum(double* rhs, const W* __restrict__ f, KP p) {
-    const long n = p.plane * (p.nz - 1);
-    const double cst = 1.0 / p.dz;
-    GRID_LOOP(t, n) {
-        const long i = p.plane + t;
-        const W d = (W)(cst * ((double)f[i + p.plane] - (double)f[i]));
-        rhs[i] = rhs[i] + (double)d;
-    }
-}
-
-template <typename W>
-void ddz_w_accum_dev(les_ctx* c, const W* f) {
-    FamScope fs(c->stream, FAM_SCALAR_FLUX, (16.0 + sizeof(W)) * (double)c->plane * (double)c->nlev);
-    KP p = kp(c);
-    hipLaunchKernelGGL(k_ddz_w_accum<W>, grid_for(p.plane * (p.nz - 1)), dim3(256), 0, c->stream,
-                       c->f3[LES_F_RHST], f, p);
 }
 
 template <typename W>
@@ -1750,7 +1841,8 @@ void max3_dev(les_ctx* c, double* out, bool lag) {
     template void wallstress_dev<W>(les_ctx*, int, const double*, const double*);                           \
     template void strain_dev<W>(les_ctx*);                                                                  \
     template void nu_t_stress_dev<W>(les_ctx*);                                                             \
-    template void ddz_w_accum_dev<W>(les_ctx*, const W*);                                                    \
+    template void scalar_flux_xy_dev<W>(les_ctx*, W*, W*);                                                  \
+    template void scalar_rhs_step_dev<W>(les_ctx*, const W*, const W*, const W*, bool, bool);               \
     template void strain_stress_dev<W>(les_ctx*);                                                           \
     template void lagrange_prep_dev<W>(les_ctx*, W*);                                                       \
     template void lagrange_contract_dev<W>(les_ctx*, const W*, const W*, int, int);                         \
@@ -1759,7 +1851,7 @@ void max3_dev(les_ctx* c, double* out, bool lag) {
     template void divstress_combine_dev<W>(les_ctx*, W*, const W*, const W*, const W*, int);                \
     template void vorticity_dev<W>(les_ctx*, W*, W*, W*);                                                   \
     template void cross_product_dev<W>(les_ctx*, const W*, const W*, const W*, W*, W*, W*);                 \
-    template void theta_prep_dev<W>(les_ctx*);                                                              \
+    template void theta_grad_dev<W>(les_ctx*);                                                              \
     template void scalar_adv_dev<W>(les_ctx*, const W*, const W*, const W*, W*);                            \
     template void scalar_flux_dev<W>(les_ctx*, W*, int);                                                    \
     template void scalar_accum_dev<W>(les_ctx*, const W*, const W*);                                        \

@@ -507,14 +507,14 @@ void theta_pre(les_ctx* c, int jt) {
     W* dtdx = WF<W>(c, LES_F_DTDX);
     W* dtdy = WF<W>(c, LES_F_DTDY);
     W* dtdz = WF<W>(c, LES_F_DTDZ);
+    swap_fields(c, LES_F_RHST, LES_F_RHST_F);   // the RHS history (:130-135)
     filter_f<double>(c, th, 0, (int)c->nlev);
     fork(c);
     level_means_seq(c->aux, th, np, 0, nz, (double)(c->nx * c->ny), c->th_mean);   // calc_hor_avg order
     les_note(c, hipEventRecord(c->ev_th, c->aux));
     ddx_f<W, double>(c, dtdx, th, 0, (int)c->nlev);
     ddy_f<W, double>(c, dtdy, th, 0, (int)c->nlev);
-    ddz_uv_dev<W, double>(c, dtdz, th);
-    theta_prep_dev<W>(c);
+    theta_grad_dev<W>(c);
     theta_pads<W>(c, dtdx, dtdy, dtdz);
 }
 
@@ -553,11 +553,11 @@ void theta_pre_overlap(les_ctx* c, int jt) {
     W* dtdx = WF<W>(c, LES_F_DTDX);
     W* dtdy = WF<W>(c, LES_F_DTDY);
     W* dtdz = WF<W>(c, LES_F_DTDZ);
+    swap_fields(c, LES_F_RHST, LES_F_RHST_F);   // the RHS history (:130-135)
     filter_f<double>(c, th, 0, (int)c->nlev);
     ddx_f<W, double>(c, dtdx, th, 0, (int)c->nlev);
     ddy_f<W, double>(c, dtdy, th, 0, (int)c->nlev);
-    ddz_uv_dev<W, double>(c, dtdz, th);
-    theta_prep_dev<W>(c);
+    theta_grad_dev<W>(c);
     theta_pads<W>(c, dtdx, dtdy, dtdz);
     level_means_seq(c->stream, th, np, 0, nz, (double)(c->nx * c->ny), c->th_mean);   // calc_hor_avg order
     les_note(c, hipEventRecord(c->ev_th, c->stream));
@@ -567,24 +567,22 @@ void theta_pre_overlap(les_ctx* c, int jt) {
 
 // advection, SGS fluxes, calc_beta and step_scalar (:466-671)
 template <typename W>
-void theta_rhs(les_ctx* c);
+void theta_advect(les_ctx* c);
+template <typename W>
+void theta_update(les_ctx* c, int jt, bool rows);
 
 template <typename W>
 void theta_post(les_ctx* c, int jt, Tape* tape = nullptr) {
-    const les_params& P = c->prm;
     const size_t np = c->plane;
     if (!theta_active(c, jt)) {
         fill_levels(c->stream, WF<W>(c, LES_F_BETA_SCAL), np, 0, (int)c->nlev, 0.0);
         return;
     }
-    theta_rhs<W>(c);
+    theta_advect<W>(c);
     les_note(c, hipStreamWaitEvent(c->stream, c->ev_th, 0));
     calc_beta_dev<W>(c, c->th_mean);
     if (tape) tape_save(c, tape, TAPE_THETA);
-    if (jt == P.theta_init_time && !P.restart_theta)
-        les_note(c, hipMemcpyAsync(F(c, LES_F_RHST_F), F(c, LES_F_RHST), np * c->nlev * 8, hipMemcpyDeviceToDevice,
-                                   c->stream));
-    step_scalar_dev(c);
+    theta_update<W>(c, jt, false);
 }
 
 // The same with theta's RHS and update on the auxiliary stream, concurrent
@@ -598,7 +596,6 @@ void theta_post(les_ctx* c, int jt, Tape* tape = nullptr) {
 // step ends.
 template <typename W>
 void theta_post_overlap(les_ctx* c, int jt, Tape* tape = nullptr) {
-    const les_params& P = c->prm;
     const size_t np = c->plane;
     if (!theta_active(c, jt)) {
         fill_levels(c->stream, WF<W>(c, LES_F_BETA_SCAL), np, 0, (int)c->nlev, 0.0);
@@ -612,22 +609,15 @@ void theta_post_overlap(les_ctx* c, int jt, Tape* tape = nullptr) {
     double** scratch[5] = {&c->work3[0], &c->work3[1], &c->work3[2], &c->work3[6], &c->big3[3]};
     std::swap(c->stream, c->aux);
     for (int i = 0; i < 5; ++i) std::swap(*scratch[i], c->tscr[i]);
-    theta_rhs<W>(c);
-    if (jt == P.theta_init_time && !P.restart_theta)
-        les_note(c, hipMemcpyAsync(F(c, LES_F_RHST_F), F(c, LES_F_RHST), np * c->nlev * 8, hipMemcpyDeviceToDevice,
-                                   c->stream));
-    step_scalar_dev(c);
-    theta_rows_dev(c);  // project's theta rows (left out of k_project_bc on the context's stream)
+    theta_advect<W>(c);
+    theta_update<W>(c, jt, true);  // with project's theta rows (left out of k_project_bc on the context's stream)
     for (int i = 0; i < 5; ++i) std::swap(*scratch[i], c->tscr[i]);
     std::swap(c->stream, c->aux);
 }
 
+// theta's advection (:466-510), into work3[2]
 template <typename W>
-void theta_fluxes(les_ctx* c, const W* adv);
-
-// theta's RHS: advection and the SGS flux divergence (:466-594)
-template <typename W>
-void theta_rhs(les_ctx* c) {
+void theta_advect(les_ctx* c) {
     const int nz = c->nz;
     const size_t np = c->plane, np2 = c->plane2;
     W* rm = scr<W>(c->big3[3]);
@@ -643,27 +633,38 @@ void theta_rhs(les_ctx* c) {
         scalar_adv_dev<W>(c, scr<W>(c->tbig[0]), scr<W>(c->tbig[1]), scr<W>(c->tbig[2]), rm);
         unpad_f<W>(c, rm + np2, adv + np, nz - 1);
     }
-    theta_fluxes<W>(c, adv);
 }
 
-// the SGS flux divergence added to the advection adv (:513-594)
+// the SGS flux divergence added to the advection (:513-594) and step_scalar;
+// rows: theta's rows 0 and nz are left as project leaves them (BOGUS)
 template <typename W>
-void theta_fluxes(les_ctx* c, const W* adv) {
-    W* temp = scr<W>(c->work3[0]);
-    W* dtemp = scr<W>(c->work3[1]);
-    scalar_flux_dev<W>(c, temp, 0);
-    ddx_f<W, W>(c, dtemp, temp, 0, (int)c->nlev);
-    scalar_accum_dev<W>(c, dtemp, adv);
-    scalar_flux_dev<W>(c, temp, 1);
-    ddy_f<W, W>(c, dtemp, temp, 0, (int)c->nlev);
-    scalar_accum_dev<W>(c, dtemp, (const W*)nullptr);
-    scalar_flux_dev<W>(c, temp, 2);
+void theta_update(les_ctx* c, int jt, bool rows) {
+    const les_params& P = c->prm;
+    const bool euler = jt == P.theta_init_time && !P.restart_theta;
+    const W* adv = scr<W>(c->work3[2]);
+    W *fx = scr<W>(c->work3[0]), *fy = scr<W>(c->work3[1]);
+    const int nl = (int)c->nlev;
     if (c->fuse) {
-        ddz_w_accum_dev<W>(c, temp);  // the vertical term added as it is differenced
-    } else {
-        ddz_w_dev<W, W>(c, dtemp, temp);
-        scalar_accum_dev<W>(c, dtemp, (const W*)nullptr);
+        scalar_flux_xy_dev<W>(c, fx, fy);
+        ddx_f<W, W>(c, fx, fx, 0, nl);
+        ddy_f<W, W>(c, fy, fy, 0, nl);
+        scalar_rhs_step_dev<W>(c, adv, fx, fy, euler, rows);
+        return;
     }
+    scalar_flux_dev<W>(c, fx, 0);
+    ddx_f<W, W>(c, fy, fx, 0, nl);
+    scalar_accum_dev<W>(c, fy, adv);
+    scalar_flux_dev<W>(c, fx, 1);
+    ddy_f<W, W>(c, fy, fx, 0, nl);
+    scalar_accum_dev<W>(c, fy, (const W*)nullptr);
+    scalar_flux_dev<W>(c, fx, 2);
+    ddz_w_dev<W, W>(c, fy, fx);
+    scalar_accum_dev<W>(c, fy, (const W*)nullptr);
+    if (euler)
+        les_note(c, hipMemcpyAsync(F(c, LES_F_RHST_F), F(c, LES_F_RHST), c->plane * c->nlev * 8,
+                                   hipMemcpyDeviceToDevice, c->stream));
+    step_scalar_dev(c);
+    if (rows) theta_rows_dev(c);
 }
 
 template <typename W>

@@ -340,7 +340,9 @@ template <typename W> void strain_dev(les_ctx* c);
 template <typename W> void lag_accumulate_dev(les_ctx* c);
 template <typename W> void nu_t_stress_dev(les_ctx* c);
 template <typename W> void strain_stress_dev(les_ctx* c);
-template <typename W> void ddz_w_accum_dev(les_ctx* c, const W* f);
+template <typename W> void scalar_flux_xy_dev(les_ctx* c, W* fx, W* fy);
+template <typename W>
+void scalar_rhs_step_dev(les_ctx* c, const W* adv, const W* dx, const W* dy, bool euler, bool rows);
 void cs_init_dev(les_ctx* c);
 template <typename W> void interpolag_dev(les_ctx* c);
 template <typename W> void lagrange_prep_dev(les_ctx* c, W* buf21);
@@ -353,7 +355,7 @@ template <typename W> void divstress_combine_dev(les_ctx* c, W* out, const W* a,
 template <typename W> void vorticity_dev(les_ctx* c, W* v1, W* v2, W* v3);
 template <typename W>
 void cross_product_dev(les_ctx* c, const W* b1, const W* b2, const W* b3, W* cx, W* cy, W* cz);
-template <typename W> void theta_prep_dev(les_ctx* c);
+template <typename W> void theta_grad_dev(les_ctx* c);
 template <typename W> void scalar_adv_dev(les_ctx* c, const W* dsx, const W* dsy, const W* dsz, W* rm);
 template <typename W> void scalar_flux_dev(les_ctx* c, W* temp, int comp);
 template <typename W> void scalar_accum_dev(les_ctx* c, const W* dtemp, const W* adv);
