@@ -6,6 +6,7 @@
 #include <utility>
 #include "fft_rg.hpp"
 #include "les_lag.hpp"
+#include "ordered_sum.hpp"
 
 namespace les {
 
@@ -142,7 +143,7 @@ void level_means(hipStream_t s, const double* f, size_t plane, int lev0, int nle
 // (theta - mean(theta) in calc_beta and the fluctuation statistics), so these
 // sums keep the reference's order.  One wavefront per sum walks the values in
 // index order, one FP64 add per value (the add's latency bounds the walk at
-// about 4 ns per value on this GPU).  The values reach it through LDS: the
+// about 3 ns per value, 10 to 14 ns beside other kernels).  The values reach it through LDS: the
 // lanes load stages of SEQ_STAGE values (coalesced) two stages ahead of the
 // walk, into a ring of three LDS stages, so a load has two stages' walking
 // time to arrive even when other kernels load the memory system.
@@ -209,41 +210,268 @@ __device__ __forceinline__ double wave_chain(long n, const F& val, double* lds) 
     return s;
 }
 
-// The walks run beside other kernels (on the auxiliary stream): at the
-// highest wave priority their dependent adds issue ahead of the other waves on
-// the SIMD instead of waiting their turn.
+// The same sum by a workgroup of OS_NT threads, for planes of more than
+// OS_MIN values: the first OS_HEAD values are walked (the sum's early binades
+// are short), then chunks of OS_NT runs of OS_RUN values are scanned
+// (ordered_sum.hpp).  A run that may leave the sum's binade is added value by
+// value and the chunk scanned again behind it; after OS_TRIES of those (sums
+// of mixed sign about zero) the rest is walked.  Bound by latency: one
+// workgroup, about 2 us a scan (a third of it the runs' roundings, the rest
+// the lane scan and the two barriers).  Obukhov's sums, walk against scan,
+// alone: 28 / 15 us at 64^2, 300 / 74 us at 256^2, 810 / 262 us at 512^2; in
+// a 512 x 512 step, beside kernels that keep the memory busy, 2600 / 818 us
+// (there the wall model waited 1.2 ms for them).  At 48^2 both take 14 us:
+// smaller planes keep the walk.
+constexpr int OS_NT = 256, OS_RUN = 16, OS_HEAD = 512, OS_TRIES = 16;
+constexpr long OS_MIN = 2048;
+constexpr int OS_NW = OS_NT / 64, OS_CHUNK = OS_NT * OS_RUN;
 
-// plane means, one wavefront (block) per plane
+struct OsLds {
+    double x[OS_CHUNK + OS_NT];   // a chunk, one padding value per run
+    double wd[OS_NW];
+    int wD[OS_NW], first[OS_NW];
+    double s;
+};
+
+// lane scan step: the map CTRL lanes below (the identity where there is none)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ SumMap dpp_map(const SumMap& m) {
+    union {
+        double d;
+        int i[2];
+    } v;
+    v.d = m.d;
+    v.i[0] = __builtin_amdgcn_update_dpp(0, v.i[0], CTRL, ROWS, 0xf, false);
+    v.i[1] = __builtin_amdgcn_update_dpp(0, v.i[1], CTRL, ROWS, 0xf, false);
+    return {v.d, __builtin_amdgcn_update_dpp(0, m.D, CTRL, ROWS, 0xf, false)};
+}
+__device__ __forceinline__ SumMap wave_scan(SumMap m) {   // inclusive
+    if (!__any(m.D != 0)) {   // no ties in this wavefront: a plain prefix sum
+        m.d += dpp_map<0x111, 0xf>(m).d;
+        m.d += dpp_map<0x112, 0xf>(m).d;
+        m.d += dpp_map<0x114, 0xf>(m).d;
+        m.d += dpp_map<0x118, 0xf>(m).d;
+        m.d += dpp_map<0x142, 0xa>(m).d;
+        m.d += dpp_map<0x143, 0xc>(m).d;
+        return m;
+    }
+    m = sum_then(dpp_map<0x111, 0xf>(m), m);   // row_shr 1, 2, 4, 8
+    m = sum_then(dpp_map<0x112, 0xf>(m), m);
+    m = sum_then(dpp_map<0x114, 0xf>(m), m);
+    m = sum_then(dpp_map<0x118, 0xf>(m), m);
+    m = sum_then(dpp_map<0x142, 0xa>(m), m);   // lane 15 of a row to the next (rows 1, 3)
+    m = sum_then(dpp_map<0x143, 0xc>(m), m);   // lane 31 to rows 2, 3
+    return m;
+}
+
+// s + the values i0..n-1 in order, walked by the first wavefront
+template <typename F>
+__device__ double block_walk(long i0, long n, const F& val, double s, OsLds& L) {
+    constexpr int ST = OS_CHUNK / 2, PER = ST / OS_NT;   // two stages
+    const int t = threadIdx.x;
+    int b = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const long i = i0 + j * OS_NT + t;
+        if (i < n) L.x[j * OS_NT + t] = val(i);
+    }
+    __syncthreads();
+    for (long base = i0; base < n; base += ST, b ^= 1) {
+        double v[PER];
+        const bool more = base + ST < n;
+        if (more) {
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                const long i = base + ST + j * OS_NT + t;
+                v[j] = val(i < n ? i : n - 1);
+            }
+        }
+        if (t < 64) {
+            // at the highest wave priority the dependent adds issue ahead of
+            // the other waves on the SIMD
+            __builtin_amdgcn_s_setprio(3);
+            const int lim = (n - base < ST) ? (int)(n - base) : ST;
+            const double* q = L.x + b * ST;
+            int j = 0;
+            for (; j + 32 <= lim; j += 32) {
+                double w[32];
+#pragma unroll
+                for (int e = 0; e < 32; ++e) w[e] = q[j + e];
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int e = 0; e < 32; ++e) s += w[e];
+            }
+            for (; j < lim; ++j) s += q[j];
+            __builtin_amdgcn_s_setprio(0);
+        }
+        if (more) {
+#pragma unroll
+            for (int j = 0; j < PER; ++j) L.x[(b ^ 1) * ST + j * OS_NT + t] = v[j];
+        }
+        __syncthreads();
+    }
+    if (t == 0) L.s = s;
+    __syncthreads();
+    return L.s;
+}
+
+template <typename F>
+__device__ double block_chain(long n, const F& val, OsLds& L) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    int tries = OS_TRIES;
+    auto load = [&](double* r, long base) {   // coalesced; s + 0 = s past the last value
+#pragma unroll
+        for (int j = 0; j < OS_RUN; ++j) {
+            const long i = base + j * OS_NT + t;
+            const double v = val(i < n ? i : n - 1);
+            r[j] = (i < n) ? v : 0.0;
+        }
+    };
+    // two chunks in flight: a load takes several us while other kernels keep
+    // the memory busy, longer than a scan
+    double n0[OS_RUN], n1[OS_RUN];
+    load(n0, OS_HEAD);
+    if (OS_HEAD + OS_CHUNK < n) load(n1, OS_HEAD + OS_CHUNK);
+    double s = block_walk(0, OS_HEAD, val, 0.0, L);
+    // adds the chunk at base, loaded in r, and refills r; true when the rest
+    // was walked
+    auto add_chunk = [&](double* r, long base) -> bool {
+        // through LDS: thread t takes the run of values OS_RUN t ..
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < OS_RUN; ++j) {
+            const int e = j * OS_NT + t;
+            L.x[e + e / OS_RUN] = r[j];
+        }
+        __syncthreads();
+        double x[OS_RUN];
+#pragma unroll
+        for (int j = 0; j < OS_RUN; ++j) x[j] = L.x[t * (OS_RUN + 1) + j];
+        if (base + 2 * OS_CHUNK < n) load(r, base + 2 * OS_CHUNK);
+        int start = 0;                              // first run not yet added
+        while (start < OS_NT) {
+            const SumGrid g = sum_grid(s);
+            const bool active = t >= start;
+            SumMap own{0.0, 0};
+            double mn = 0.0, mx = 0.0;
+            if (active) own = sum_run<OS_RUN>(x, g, mn, mx);
+            const SumMap m = wave_scan(own);
+            SumMap ex{__shfl_up(m.d, 1), __shfl_up(m.D, 1)};
+            if (lane == 0) ex = SumMap{0.0, 0};
+            if (lane == 63) {
+                L.wd[wave] = m.d;
+                L.wD[wave] = m.D;
+            }
+            __syncthreads();
+            SumMap all{0.0, 0}, pre{0.0, 0};
+#pragma unroll
+            for (int q = 0; q < OS_NW; ++q) {
+                if (q == wave) pre = all;
+                all = sum_then(all, SumMap{L.wd[q], L.wD[q]});
+            }
+            const double at = sum_add(sum_then(pre, ex), g.odd);
+            const unsigned long long out = __ballot(active && !sum_inside(g, at, own, mn, mx));
+            if (lane == 0) L.first[wave] = out ? wave * 64 + __ffsll(out) - 1 : OS_NT;
+            __syncthreads();
+            int stop = OS_NT;
+#pragma unroll
+            for (int q = 0; q < OS_NW; ++q) stop = min(stop, L.first[q]);
+            if (stop == OS_NT) {
+                s = sum_value(g, s, sum_add(all, g.odd));
+                return false;
+            }
+            if (t == stop) {
+                double v = sum_value(g, s, at);
+#pragma unroll
+                for (int j = 0; j < OS_RUN; ++j) v += x[j];
+                L.s = v;
+            }
+            __syncthreads();
+            s = L.s;
+            start = stop + 1;
+            if (--tries == 0) {
+                __syncthreads();
+                s = block_walk(base + (long)start * OS_RUN, n, val, s, L);
+                return true;
+            }
+        }
+        return false;
+    };
+    for (long base = OS_HEAD; base < n; base += 2 * OS_CHUNK) {
+        if (add_chunk(n0, base)) break;
+        if (base + OS_CHUNK < n && add_chunk(n1, base + OS_CHUNK)) break;
+    }
+    return s;
+}
+
+// plane means, one workgroup per plane
 __global__ __launch_bounds__(64) void k_level_means_seq(const double* __restrict__ f, long plane, double nn,
                                                          double* __restrict__ out) {
+    // at the highest wave priority the walk's dependent adds issue ahead of
+    // the other waves on the SIMD
     __builtin_amdgcn_s_setprio(3);
     __shared__ __align__(16) double lds[3 * SEQ_STAGE];
     const double* p = f + (long)blockIdx.x * plane;
     const double s = wave_chain(plane, [&](long i) { return p[i]; }, lds);
     if (threadIdx.x == 0) out[blockIdx.x] = s / nn;
 }
+__global__ __launch_bounds__(OS_NT) void k_level_means_scan(const double* __restrict__ f, long plane, double nn,
+                                                            double* __restrict__ out) {
+    __shared__ OsLds L;
+    const double* p = f + (long)blockIdx.x * plane;
+    const double s = block_chain(plane, [&](long i) { return p[i]; }, L);
+    if (threadIdx.x == 0) out[blockIdx.x] = s / nn;
+}
 
 void level_means_seq(hipStream_t s, const double* f, size_t plane, int lev0, int nlev, double nn, double* out) {
     FamScope fs(s, FAM_PLANE_SUMS, 8.0 * (double)plane * nlev);
-    hipLaunchKernelGGL(k_level_means_seq, dim3(nlev), dim3(64), 0, s, f + (size_t)lev0 * plane, (long)plane, nn,
-                       out);
+    const double* p = f + (size_t)lev0 * plane;
+    if ((long)plane > OS_MIN)
+        hipLaunchKernelGGL(k_level_means_scan, dim3(nlev), dim3(OS_NT), 0, s, p, (long)plane, nn, out);
+    else
+        hipLaunchKernelGGL(k_level_means_seq, dim3(nlev), dim3(64), 0, s, p, (long)plane, nn, out);
 }
 
-// obukhov sums at the wall level, in the reference's order, one wavefront
+// obukhov sums at the wall level, in the reference's order, one workgroup
 // per sum: [0] sum sqrt(u^2+v^2), [1] sum psi_m, [2] sum sgs_t3(1), [3] sum theta(1)
+template <typename SUM>
+__device__ __forceinline__ void obukhov_sums(const SUM& sum, const double* __restrict__ u1,
+                                             const double* __restrict__ v1, const double* __restrict__ psi,
+                                             const double* __restrict__ t3, const double* __restrict__ th1,
+                                             double* __restrict__ out) {
+    const int which = blockIdx.x;
+    double s;
+    if (which == 0) {
+        s = sum([&](long i) { return sqrt(u1[i] * u1[i] + v1[i] * v1[i]); });
+    } else {
+        const double* __restrict__ p = which == 1 ? psi : (which == 2 ? t3 : th1);
+        s = sum([&](long i) { return p[i]; });
+    }
+    if (threadIdx.x == 0) out[which] = s;
+}
 __global__ __launch_bounds__(64) void k_obukhov_sums(const double* __restrict__ u1, const double* __restrict__ v1,
                                                       const double* __restrict__ psi, const double* __restrict__ t3,
                                                       const double* __restrict__ th1, long plane,
                                                       double* __restrict__ out) {
     __builtin_amdgcn_s_setprio(3);
     __shared__ __align__(16) double lds[3 * SEQ_STAGE];
-    const int which = blockIdx.x;
-    double s;
-    if (which == 0) s = wave_chain(plane, [&](long i) { return sqrt(u1[i] * u1[i] + v1[i] * v1[i]); }, lds);
-    else if (which == 1) s = wave_chain(plane, [&](long i) { return psi[i]; }, lds);
-    else if (which == 2) s = wave_chain(plane, [&](long i) { return t3[i]; }, lds);
-    else s = wave_chain(plane, [&](long i) { return th1[i]; }, lds);
-    if (threadIdx.x == 0) out[which] = s;
+    obukhov_sums([&](const auto& val) { return wave_chain(plane, val, lds); }, u1, v1, psi, t3, th1, out);
+}
+__global__ __launch_bounds__(OS_NT) void k_obukhov_sums_scan(const double* __restrict__ u1,
+                                                             const double* __restrict__ v1,
+                                                             const double* __restrict__ psi,
+                                                             const double* __restrict__ t3,
+                                                             const double* __restrict__ th1, long plane,
+                                                             double* __restrict__ out) {
+    __shared__ OsLds L;
+    obukhov_sums([&](const auto& val) { return block_chain(plane, val, L); }, u1, v1, psi, t3, th1, out);
+}
+static void launch_obukhov_sums(hipStream_t s, int nsums, const double* u1, const double* v1, const double* psi,
+                                const double* t3, const double* th1, long plane, double* out) {
+    if (plane > OS_MIN)
+        hipLaunchKernelGGL(k_obukhov_sums_scan, dim3(nsums), dim3(OS_NT), 0, s, u1, v1, psi, t3, th1, plane, out);
+    else
+        hipLaunchKernelGGL(k_obukhov_sums, dim3(nsums), dim3(64), 0, s, u1, v1, psi, t3, th1, plane, out);
 }
 
 // neutral / theta-off branch, 010_scalars.f90:718-738
@@ -311,15 +539,13 @@ void obukhov_sums_dev(les_ctx* c, int jt, hipStream_t s) {
         // the surface ranks' planes are left as they are; the top wall's
         // ranks take their ustar_avg from level nz-1
         if (P.ubc_mom == LES_BC_WALL)
-            hipLaunchKernelGGL(k_obukhov_sums, dim3(1), dim3(64), 0, s, u1 + (long)(c->nz - 2) * np,
-                               v1 + (long)(c->nz - 2) * np, (const double*)nullptr, (const double*)nullptr,
-                               (const double*)nullptr, np, c->red);
+            launch_obukhov_sums(s, 1, u1 + (long)(c->nz - 2) * np, v1 + (long)(c->nz - 2) * np, nullptr, nullptr,
+                                nullptr, np, c->red);
         return;
     }
     if (!P.theta_flag || jt < P.theta_init_time) {
         if (!P.restart_theta) fill_levels(s, c->psi_m, c->plane, 0, 1, 0.0);
-        hipLaunchKernelGGL(k_obukhov_sums, dim3(2), dim3(64), 0, s, u1, v1, c->psi_m, (const double*)nullptr,
-                           (const double*)nullptr, np, c->red);
+        launch_obukhov_sums(s, 2, u1, v1, c->psi_m, nullptr, nullptr, np, c->red);
         return;
     }
     double* t3 = c->f3[LES_F_SGS_T3] + np;
@@ -327,8 +553,7 @@ void obukhov_sums_dev(les_ctx* c, int jt, hipStream_t s) {
         fill_levels(s, t3, c->plane, 0, 1, P.wt_s / P.u_scale / P.T_scale);
     // theta(1) as the previous step left it: a copy taken on the context's
     // stream, since the step filters theta while these sums may still run
-    hipLaunchKernelGGL(k_obukhov_sums, dim3(4), dim3(64), 0, s, u1, v1, c->psi_m, (const double*)t3,
-                       (const double*)c->th1_copy, np, c->red);
+    launch_obukhov_sums(s, 4, u1, v1, c->psi_m, t3, c->th1_copy, np, c->red);
 }
 
 // the rest of obukhov from the sums, on the context's stream
