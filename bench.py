@@ -297,20 +297,20 @@ _POINT_FAMILIES = [
     (("k_scalar_flux", "k_scalar_accum", "k_scalar_rhs_step"), "scalar_flux"),
     (("k_ddz_uv", "k_ddz_w<", "k_theta_grad"), "ddz"),
     (("k_divstress",), "divstress"),
-    (("k_max3_lag", "k_max3_part", "k_max3_final"), "cfl_max"),
+    (("k_step_begin", "k_max3_part", "k_max3_final"), "cfl_max"),
     (("k_press_prep", "k_dpdz", "k_hz_part", "k_hz_fold"), "press_prep"),
     (("k_lag_prep", "k_interpolag", "k_lag_contract<", "k_lag_acc"), "lagrange_point"),
     (("k_step_scalar", "k_calc_beta", "k_scalar_top"), "theta_point"),
     (("k_tdma",), "tdma"),
     (("kr_lag_contract",), "lag_contract_x"),
-    (("kr_x_r2c", "k_x_r2c"), "x_r2c"),
+    (("kr_x_r2c", "k_x_r2c", "kr_x_press"), "x_r2c"),
     (("kr_x_c2r", "k_x_c2r"), "x_c2r"),
     (("kr_yspec", "k_yline_spec"), "yline.spec"),
     (("k_vort<",), "vort_pad_x"),
 ]
 # the first kernel of every step: obukhov's plane sums, which les_run launches
 # before the CFL pass, or the CFL pass where a step has no such sums
-_STEP_START = (("k_obukhov_sums",), ("k_max3_lag", "k_max3_part"))
+_STEP_START = (("k_obukhov_sums",), ("k_step_begin", "k_max3_part"))
 # kernels that follow another one inside the same bracket of les_profile_step,
 # so that a family's launches count brackets, as the library's profiler does
 _SECONDARY = ("k_project_bc", "k_max3_final", "k_scalar_top", "k_hz_fold")

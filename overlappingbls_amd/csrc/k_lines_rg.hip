@@ -96,6 +96,17 @@ bool yline_spec_ct(hipStream_t s, const Batch<cx<T>, cx<T>>& io, int nplanes, in
     return true;
 }
 
+bool press_x_available(const Twiddle& tw) { return g_use_ct && rg_table(tw.n) != nullptr; }
+template <typename W>
+void press_x(hipStream_t s, const PressIn<W>& a, bool filter, const Twiddle& tw) {
+    // u, v, w read, three half spectra written, and with filter u, v, w written
+    FamScope fs(s, FAM_XR2C,
+                3.0 * (a.nz - 1) * a.ny * (8.0 * tw.n * (filter ? 2.0 : 1.0) + sizeof(W) * (tw.n + 2.0)));
+    rg_ops<W>(rg_table(tw.n)).press(s, a, filter, tw);
+}
+template void press_x<double>(hipStream_t, const PressIn<double>&, bool, const Twiddle&);
+template void press_x<float>(hipStream_t, const PressIn<float>&, bool, const Twiddle&);
+
 template <typename T>
 bool cross_unpad_x(hipStream_t s, const ConvIn<T>& a, int scalar, T* o0, T* o1, T* o2, int nz, int ny2,
                    const Twiddle& tin, const Twiddle& tout) {

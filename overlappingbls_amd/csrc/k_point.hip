@@ -3,6 +3,7 @@
 // 0..nzt; the bottom z-slab's rules at levels 0/1, the top z-slab's at
 // nzt-1/nzt).  Streaming kernels are HBM-bound: one read of each input and
 // one write of each output per point, grid-stride over (level, plane).
+#include <algorithm>
 #include <utility>
 #include "fft_rg.hpp"
 #include "les_lag.hpp"
@@ -1707,6 +1708,7 @@ struct RhsOpts {
     const double *ust, *vst;  // Stokes drift (0:nz)
     const double* mn;         // plane means of u, v, w at levels 1..nz-1 (mn[k-1], mn[nlev+k-1], ...)
     long nlev;
+    double* shift;            // the advanced u, v, w of each level's first point (3 nlev)
 };
 
 // RHS assembly (103_flosol.f90:115-157) fused with Admas_Bashforth
@@ -1769,9 +1771,17 @@ __global__ void k_rhs_ab2(RhsArgs<W> a, double* u, double* v, double* w, KP p, R
         } else {
             rxf = (double)a.rxf[i]; ryf = (double)a.ryf[i]; rzf = (double)a.rzf[i];
         }
-        u[i] = u[i] + p.dt * (tadv1 * rx + tadv2 * rxf + 0.0 + o.force);
-        v[i] = v[i] + p.dt * (tadv1 * ry + tadv2 * ryf + 0.0);
-        w[i] = w[i] + p.dt * (tadv1 * rz + tadv2 * rzf + 0.0);
+        const double un = u[i] + p.dt * (tadv1 * rx + tadv2 * rxf + 0.0 + o.force);
+        const double vn = v[i] + p.dt * (tadv1 * ry + tadv2 * ryf + 0.0);
+        const double wn = w[i] + p.dt * (tadv1 * rz + tadv2 * rzf + 0.0);
+        u[i] = un;
+        v[i] = vn;
+        w[i] = wn;
+        if (i == (long)k * p.plane) {
+            o.shift[k] = un;
+            o.shift[o.nlev + k] = vn;
+            o.shift[2 * o.nlev + k] = wn;
+        }
     }
 }
 
@@ -1807,6 +1817,7 @@ void rhs_ab2_dev(les_ctx* c, int jt) {
     o.ust = c->ust; o.vst = c->vst;
     o.mn = c->dmean;
     o.nlev = (long)c->nlev;
+    o.shift = c->shift;
     if (o.damp23) {
         // calc_hor_avg3 of u, v, w at levels 1..nz-1 (007_topbc.f90:110-112), in order
         const double nn = (double)(c->nx * c->ny);
@@ -1849,16 +1860,20 @@ void ab2_dev(les_ctx* c) {
 // RHS -= grad p (103_flosol.f90:179-181; the dudt diagnostics likewise,
 // :183-185, when du != null) fused with project (110_project.f90:16-40):
 // u, v on levels 1..nz-1, w from level 2
+// dp/dz is formed here from p (rounded to W as k_dpdz stores it) and written
+// for the caller, one field read less than behind k_dpdz.
 template <typename W>
 __global__ void k_gradp_project(W* rx, W* ry, W* rz, double* u, double* v, double* w,
-                                const W* __restrict__ px, const W* __restrict__ py, const W* __restrict__ pz, KP p,
-                                double* du, double* dv, double* dw) {
+                                const W* __restrict__ px, const W* __restrict__ py, const W* __restrict__ pr, W* pz,
+                                KP p, double* du, double* dv, double* dw) {
     const long n = p.plane * (p.nz - 1);
     const double tadv1 = 1.5;
     GRID_LOOP(t, n) {
         const long i = p.plane + t;
         const int k = (int)(i / p.plane);
-        const double gx = px[i], gy = py[i], gz = pz[i];
+        const W dz = (W)(((double)pr[i] - (double)pr[i - p.plane]) / p.dz);
+        pz[i] = dz;
+        const double gx = px[i], gy = py[i], gz = dz;
         rx[i] = (W)((double)rx[i] - gx);
         ry[i] = (W)((double)ry[i] - gy);
         rz[i] = (W)((double)rz[i] - gz);
@@ -1926,15 +1941,15 @@ void theta_rows_dev(les_ctx* c) {
 // theta_rows = false: theta's rows are left to theta_rows_dev
 template <typename W>
 void gradp_project_dev(les_ctx* c, int jt, bool theta_rows) {
-    // RHS (work precision) read and written, u, v, w read and written, grad p read
-    FamScope fs(c->stream, FAM_GRADP_PROJECT, (48.0 + 9.0 * sizeof(W)) * (double)c->plane * (c->nz - 1));
+    // RHS (work precision) and u, v, w read and written, p, dp/dx, dp/dy read, dp/dz written
+    FamScope fs(c->stream, FAM_GRADP_PROJECT, (48.0 + 10.0 * sizeof(W)) * (double)c->plane * (c->nz - 1));
     KP p = kp(c);
     const les_params& P = c->prm;
     const bool st = stats_step(c, jt);
     hipLaunchKernelGGL(k_gradp_project<W>, grid_for(p.plane * (p.nz - 1)), dim3(256), 0, c->stream,
                        WF<W>(c, LES_F_RHSX), WF<W>(c, LES_F_RHSY), WF<W>(c, LES_F_RHSZ), c->f3[LES_F_U], c->f3[LES_F_V],
                        c->f3[LES_F_W], (const W*)WF<W>(c, LES_F_DPDX), (const W*)WF<W>(c, LES_F_DPDY),
-                       (const W*)WF<W>(c, LES_F_DPDZ), p, st ? c->st_diag[0] : nullptr,
+                       (const W*)WF<W>(c, LES_F_P), WF<W>(c, LES_F_DPDZ), p, st ? c->st_diag[0] : nullptr,
                        st ? c->st_diag[1] : nullptr, st ? c->st_diag[2] : nullptr);
     hipLaunchKernelGGL(k_project_bc, grid_for(p.plane), dim3(256), 0, c->stream, c->f3[LES_F_U], c->f3[LES_F_V],
                        c->f3[LES_F_W], c->f3[LES_F_THETA], p, (int)(P.ubc_mom == LES_BC_STRESS_FREE),
@@ -1982,20 +1997,36 @@ __global__ __launch_bounds__(256) void k_max3_part(const double* __restrict__ u,
         for (int a = 0; a < 3; ++a) part[a * MAXB + blockIdx.x] = sh[a][0];
 }
 
-// k_max3_part over levels lo..hi fused with k_lag_acc over all n values:
-// u, v, w are read once
-template <typename W>
-__global__ __launch_bounds__(256) void k_max3_lag(const double* __restrict__ u, const double* __restrict__ v,
-                                                  const double* __restrict__ w, W* ul, W* vl, W* wl,
-                                                  long n, long lo, long hi, double* __restrict__ part) {
+// The passes over u, v, w that open a step in one: check_cfl's partial maxima
+// (k_max3_part, levels 1..nz-1), the vertical differences (k_ddz_uvw) and,
+// with LAG, sgs_stag's u_lag accumulation (k_lag_acc, all levels).  Twelve
+// field passes instead of fifteen; bound by HBM.
+template <typename W, bool LAG>
+__global__ __launch_bounds__(256) void k_step_begin(const double* __restrict__ u, const double* __restrict__ v,
+                                                    const double* __restrict__ w, W* ul, W* vl, W* wl, W* uz, W* vz,
+                                                    W* wz, KP p, double* __restrict__ part) {
     __shared__ double sh[3][256];
     double m[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
+    const long n = p.plane * (p.nz + 1);
+    const double cst = 1.0 / p.dz;
+    GRID_LOOP(i, n) {
+        const int k = (int)(i / p.plane);
         const double a = u[i], b = v[i], d = w[i];
-        ul[i] = (W)((double)ul[i] + a);
-        vl[i] = (W)((double)vl[i] + b);
-        wl[i] = (W)((double)wl[i] + d);
-        if (i >= lo && i < hi) {
+        if constexpr (LAG) {
+            ul[i] = (W)((double)ul[i] + a);
+            vl[i] = (W)((double)vl[i] + b);
+            wl[i] = (W)((double)wl[i] + d);
+        }
+        if (k == 0) {
+            uz[i] = BOGUS; vz[i] = BOGUS; wz[i] = BOGUS;
+        } else if (k == p.nz) {
+            wz[i] = 0.0;
+        } else {
+            if (k >= 2) {
+                uz[i] = cst * (a - u[i - p.plane]);
+                vz[i] = cst * (b - v[i - p.plane]);
+            }
+            wz[i] = cst * (w[i + p.plane] - d);
             m[0] = fmax(m[0], a);
             m[1] = fmax(m[1], b);
             m[2] = fmax(m[2], d);
@@ -2034,31 +2065,45 @@ __global__ __launch_bounds__(256) void k_max3_final(const double* __restrict__ p
     if (threadIdx.x == 0) *out = sh[0][0] * cu + sh[1][0] * cv + sh[2][0] * cw;
 }
 
-void max3_dev(les_ctx* c, double* out, bool lag) {
-    const bool m32 = c->precision == LES_MIXED;  // u_lag in the work precision
-    FamScope fs(c->stream, FAM_CFL_MAX,
-                (24.0 + (lag ? 6.0 * (m32 ? 4.0 : 8.0) : 0.0)) * (double)c->plane * (double)c->nlev);
-    const long lo = (long)c->plane, hi = (long)c->plane * c->nz;
-    const long n = lag ? (long)c->plane * (long)c->nlev : hi - lo;
-    long nb = (n + 255) / 256;
-    if (nb > MAXB) nb = MAXB;
+static void max3_final(les_ctx* c, const double* part, long nb, double* out) {
     const double dt = c->prm.dt;
+    hipLaunchKernelGGL(k_max3_final, dim3(1), dim3(256), 0, c->stream, part, (int)nb, out, dt / c->dx, dt / c->dy,
+                       dt / c->dz);
+}
+
+void max3_dev(les_ctx* c, double* out) {
+    FamScope fs(c->stream, FAM_CFL_MAX, 24.0 * (double)c->plane * (double)c->nlev);
+    const long lo = (long)c->plane, hi = (long)c->plane * c->nz;
+    const long nb = std::min((hi - lo + 255) / 256, (long)MAXB);
     double* part = c->red + 64;  // red holds >= 64 + 3*MAXB doubles
-    if (lag && m32)
-        hipLaunchKernelGGL(k_max3_lag<float>, dim3((unsigned)nb), dim3(256), 0, c->stream,
-                           (const double*)c->f3[LES_F_U], (const double*)c->f3[LES_F_V],
-                           (const double*)c->f3[LES_F_W], WF<float>(c, LES_F_U_LAG), WF<float>(c, LES_F_V_LAG),
-                           WF<float>(c, LES_F_W_LAG), n, lo, hi, part);
-    else if (lag)
-        hipLaunchKernelGGL(k_max3_lag<double>, dim3((unsigned)nb), dim3(256), 0, c->stream,
-                           (const double*)c->f3[LES_F_U], (const double*)c->f3[LES_F_V],
-                           (const double*)c->f3[LES_F_W], WF<double>(c, LES_F_U_LAG), WF<double>(c, LES_F_V_LAG),
-                           WF<double>(c, LES_F_W_LAG), n, lo, hi, part);
+    hipLaunchKernelGGL(k_max3_part, dim3((unsigned)nb), dim3(256), 0, c->stream, (const double*)c->f3[LES_F_U],
+                       (const double*)c->f3[LES_F_V], (const double*)c->f3[LES_F_W], lo, hi, part);
+    max3_final(c, part, nb, out);
+}
+
+template <typename W>
+void step_begin_dev(les_ctx* c, double* out, bool lag) {
+    FamScope fs(c->stream, FAM_CFL_MAX,
+                (24.0 + (lag ? 9.0 : 3.0) * sizeof(W)) * (double)c->plane * (double)c->nlev);
+    const KP p = kp(c);
+    const long nb = std::min((p.plane * (p.nz + 1) + 255) / 256, (long)MAXB);
+    double* part = c->red + 64;
+    const double *u = c->f3[LES_F_U], *v = c->f3[LES_F_V], *w = c->f3[LES_F_W];
+    W *ul = WF<W>(c, LES_F_U_LAG), *vl = WF<W>(c, LES_F_V_LAG), *wl = WF<W>(c, LES_F_W_LAG);
+    W *uz = WF<W>(c, LES_F_DUDZ), *vz = WF<W>(c, LES_F_DVDZ), *wz = WF<W>(c, LES_F_DWDZ);
+    if (lag)
+        hipLaunchKernelGGL((k_step_begin<W, true>), dim3((unsigned)nb), dim3(256), 0, c->stream, u, v, w, ul, vl, wl, uz, vz,
+                           wz, p, part);
     else
-        hipLaunchKernelGGL(k_max3_part, dim3((unsigned)nb), dim3(256), 0, c->stream, (const double*)c->f3[LES_F_U],
-                           (const double*)c->f3[LES_F_V], (const double*)c->f3[LES_F_W], lo, hi, part);
-    hipLaunchKernelGGL(k_max3_final, dim3(1), dim3(256), 0, c->stream, (const double*)part, (int)nb, out,
-                       dt / c->dx, dt / c->dy, dt / c->dz);
+        hipLaunchKernelGGL((k_step_begin<W, false>), dim3((unsigned)nb), dim3(256), 0, c->stream, u, v, w, ul, vl, wl, uz, vz,
+                           wz, p, part);
+    max3_final(c, part, nb, out);
+}
+
+// lbc = 0's surface-temperature term taken off Hz(0)'s mean coefficient
+__global__ void k_press_modi(cx<double>* h, double modi) { h[0].x = h[0].x - modi; }
+void press_modi_dev(les_ctx* c, cx<double>* h, double modi) {
+    hipLaunchKernelGGL(k_press_modi, dim3(1), dim3(1), 0, c->stream, h, modi);
 }
 
 // ---- instantiations for both work precisions --------------------------------
@@ -2087,6 +2132,7 @@ void max3_dev(les_ctx* c, double* out, bool lag) {
     template void dpdz_on<W>(les_ctx*, W*, const W*);                                                       \
     template void press_hz_sums_dev<W>(les_ctx*, double*, double);                                          \
     template void dpdz_dev<W>(les_ctx*);                                                                    \
+    template void step_begin_dev<W>(les_ctx*, double*, bool);                                               \
     template void rhs_ab2_dev<W>(les_ctx*, int);                                                            \
     template void lag_accumulate_dev<W>(les_ctx*);                                                          \
     template void interpolag_dev<W>(les_ctx*);                                                              \

@@ -17,6 +17,22 @@ using namespace les;
 
 namespace les {
 
+// From the right-hand sides' spectra (spec3[0..2] after the y transforms; the
+// mixed mode's mean column in hzm) to p, dp/dx, dp/dy
+template <typename W>
+static void press_spectra(les_ctx* c, W* pf, W* dpdx, W* dpdy) {
+    const int nz = c->nz;
+    const size_t np = c->plane, ns = c->ns;
+    cx<W>*Hx = scr<W>(c->spec3[0]), *Hy = scr<W>(c->spec3[1]), *Hz = scr<W>(c->spec3[2]);
+    const bool m = sizeof(W) < sizeof(double);
+    cx<W>* ph = m ? reinterpret_cast<cx<W>*>(c->phf) : scr<W>(c->spec3[3]);
+    tdma_press<W>(c, Hx, Hy, Hz, ph, reinterpret_cast<double*>(c->spec3[3]), m ? c->hzm : nullptr);
+    yline_spec<W>(c->stream, ph, ph, nz, c->lhx, (long)ns, c->tw_y, SP_INV, nullptr);
+    x_c2r<W>(c->stream, ph, pf, (long)nz * c->ny, c->lhx, c->nx, c->tw_x, 0, 0.0);
+    x_c2r<W>(c->stream, ph + ns, dpdx + np, (long)(nz - 1) * c->ny, c->lhx, c->nx, c->tw_x, 1, kfx(c));
+    ddy_f<W, W>(c, dpdy, pf, 1, nz - 1);
+}
+
 // press_stag_array (109_press_stag_array.f90:104-238) on explicit fields:
 // (u, v, w, divtz(1), divtz(nz)) -> p (levels 0..nz-1), dp/dx, dp/dy, dp/dz
 // (levels 1..nz-1).  Linear in its inputs; the linearised step calls it on
@@ -33,20 +49,8 @@ void press_solve(les_ctx* c, const double* u, const double* v, const double* w, 
     x_r2c<W, W>(c->stream, batch3<cx<W>, W>(rx, ry, rz, Hx, Hy, Hz), rows, c->nx, c->lhx, c->tw_x, 1.0);
     yline_spec<W>(c->stream, batch3<cx<W>, cx<W>>(Hx, Hy, Hz, Hx, Hy, Hz), nz + 1, c->lhx, (long)ns, c->tw_y, SP_FWD,
                   nullptr);
-    cx<W>* ph;
-    const double* hzm = nullptr;
-    if (sizeof(W) == sizeof(double)) {
-        ph = scr<W>(c->spec3[3]);
-    } else {
-        ph = reinterpret_cast<cx<W>*>(c->phf);
-        press_hz_sums_dev<W>(c, c->hzm, modi);
-        hzm = c->hzm;
-    }
-    tdma_press<W>(c, Hx, Hy, Hz, ph, reinterpret_cast<double*>(c->spec3[3]), hzm);
-    yline_spec<W>(c->stream, ph, ph, nz, c->lhx, (long)ns, c->tw_y, SP_INV, nullptr);
-    x_c2r<W>(c->stream, ph, pf, (long)nz * c->ny, c->lhx, c->nx, c->tw_x, 0, 0.0);
-    x_c2r<W>(c->stream, ph + ns, dpdx + np, (long)(nz - 1) * c->ny, c->lhx, c->nx, c->tw_x, 1, kfx(c));
-    ddy_f<W, W>(c, dpdy, pf, 1, nz - 1);
+    if (sizeof(W) < sizeof(double)) press_hz_sums_dev<W>(c, c->hzm, modi);
+    press_spectra<W>(c, pf, dpdx, dpdy);
     dpdz_on<W>(c, dpdz, pf);
 }
 template void press_solve<double>(les_ctx*, const double*, const double*, const double*, const double*, double*,
@@ -68,6 +72,8 @@ double press_modi(const les_ctx* c, int jt) {
 }  // namespace les
 
 namespace {
+
+bool mixed(const les_ctx* c) { return c->precision == LES_MIXED; }
 
 int good_size(int n) {
     if (n < 8 || n % 4) return 0;
@@ -729,6 +735,47 @@ void obukhov_sums_fork(les_ctx* c, int jt) {
     les_note(c, hipEventRecord(c->ev_obk, c->sums));
 }
 
+// The step's pressure solve, projection and filter_data of u, v, w.  In FP64
+// the filter is taken in front of the projection (kr_x_press): its x pass
+// shares the row transforms of the pressure's right-hand side, and its y pass
+// runs on the third stream beside the solve, whose column sweeps leave the
+// memory idle.  The mixed mode's single-precision pressure gradient carries
+// rounding in its Nyquist modes, so there the filter stays behind the
+// projection.  Not on statistics steps, which sample the unfiltered projected
+// velocity (diagnostics_ke).
+template <typename W>
+void press_filter_project(les_ctx* c, int jt, bool theta_rows) {
+    const int nz = c->nz;
+    const size_t np = c->plane, ns = c->ns;
+    const double modi = press_modi(c, jt);
+    const W* divtz = WF<W>(c, LES_F_DIVTZ);
+    double *u = F(c, LES_F_U), *v = F(c, LES_F_V), *w = F(c, LES_F_W);
+    cx<W>*Hx = scr<W>(c->spec3[0]), *Hy = scr<W>(c->spec3[1]), *Hz = scr<W>(c->spec3[2]);
+    const double cst = 1.0 / (double)(c->nx * c->ny);
+    if (mixed(c)) press_hz_sums_dev<W>(c, c->hzm, modi);   // reads w before it is filtered
+    const PressIn<W> a{u, v, w, divtz + np, divtz + (size_t)nz * np, Hx, Hy, Hz, c->shift, c->ny, nz,
+                       cst / 1.5 / c->prm.dt, cst};
+    const bool before = !mixed(c);   // filter in front of the projection
+    press_x<W>(c->stream, a, before && c->fuse, c->tw_x);
+    if (before) {
+        const Batch<double, double> fb = batch3<double, double>(u + np, v + np, w + np, u + np, v + np, w + np);
+        if (!c->fuse)
+            xline_real<double>(c->stream, fb, (long)(nz - 1) * c->ny, c->nx, c->nx, c->tw_x, c->tw_x, OP_NYQ, 0.0);
+        les_note(c, hipEventRecord(c->ev_xf, c->stream));
+        les_note(c, hipStreamWaitEvent(c->sums, c->ev_xf, 0));
+        yline_real<double>(c->sums, fb, nz - 1, c->nx, c->nx, c->nx, (long)np, (long)np, c->tw_y, c->tw_y, OP_NYQ,
+                           0.0);
+        les_note(c, hipEventRecord(c->ev_yf, c->sums));
+    }
+    yline_spec<W>(c->stream, batch3<cx<W>, cx<W>>(Hx, Hy, Hz, Hx, Hy, Hz), nz + 1, c->lhx, (long)ns, c->tw_y, SP_FWD,
+                  nullptr);
+    if (modi != 0.0 && !mixed(c)) press_modi_dev(c, c->spec3[2], modi);
+    press_spectra<W>(c, WF<W>(c, LES_F_P), WF<W>(c, LES_F_DPDX), WF<W>(c, LES_F_DPDY));
+    if (before) les_note(c, hipStreamWaitEvent(c->stream, c->ev_yf, 0));
+    gradp_project_dev<W>(c, jt, theta_rows);
+    if (!before) filter3_f(c, u, v, w, (int)c->nlev);
+}
+
 template <typename W>
 void step_body(les_ctx* c, int jt, Tape* tape = nullptr, bool stats = true) {
     // newstep: RHS_f = RHS (103_flosol.f90:311-313) as a pointer exchange
@@ -749,7 +796,8 @@ void step_body(les_ctx* c, int jt, Tape* tape = nullptr, bool stats = true) {
     ddy3_f<W, double>(c,
                       batch3<W, double>(u, v, w, WF<W>(c, LES_F_DUDY), WF<W>(c, LES_F_DVDY), WF<W>(c, LES_F_DWDY)), 0,
                       nl);
-    ddz_uvw_dev<W>(c);
+    if (!c->ddz_done) ddz_uvw_dev<W>(c);
+    c->ddz_done = 0;
     // theta's filter, gradients and pads: on aux (submitted after the
     // derivatives, so that the host, which has a bounded number of launches
     // outstanding, hands the momentum stream its work first), or in order
@@ -767,16 +815,19 @@ void step_body(les_ctx* c, int jt, Tape* tape = nullptr, bool stats = true) {
     if (ovl) theta_post_overlap<W>(c, jt, tape);
     else theta_post<W>(c, jt, tape);
     rhs_ab2_dev<W>(c, jt);
-    press_stag_array<W>(c, jt);
-    gradp_project_dev<W>(c, jt, !(ovl && theta_active(c, jt)));
-    if (st) diagnostics_ke(c);
-    filter3_f(c, F(c, LES_F_U), F(c, LES_F_V), F(c, LES_F_W), nl);
+    const bool theta_rows = !(ovl && theta_active(c, jt));
+    if (!st && press_x_available(c->tw_x)) {
+        press_filter_project<W>(c, jt, theta_rows);
+    } else {
+        press_stag_array<W>(c, jt);
+        gradp_project_dev<W>(c, jt, theta_rows);
+        if (st) diagnostics_ke(c);
+        filter3_f(c, F(c, LES_F_U), F(c, LES_F_V), F(c, LES_F_W), nl);
+    }
     if (ovl) join(c);
     if (st) avg_slices<W>(c, jt);
     if (tape) tape_save(c, tape, TAPE_END);
 }
-
-bool mixed(const les_ctx* c) { return c->precision == LES_MIXED; }
 
 // Run a routine templated on the work precision in the current mode.
 #define LES_DISPATCH(fn, ...)                          \
@@ -1030,7 +1081,9 @@ int les_create(const les_params* prm, les_ctx** out) {
         hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->ev_obk, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->ev_th, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->ev_uvw, hipEventDisableTiming) != hipSuccess) {
+        hipEventCreateWithFlags(&c->ev_uvw, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&c->ev_xf, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&c->ev_yf, hipEventDisableTiming) != hipSuccess) {
         les_destroy(c);
         return LES_E_HIP;
     }
@@ -1040,6 +1093,7 @@ int les_create(const les_params* prm, les_ctx** out) {
     double** surfs[6] = {&c->ustar, &c->psi_m, &c->phi_m, &c->psi_h, &c->phi_h, &c->ustar_top};
     for (int s = 0; s < 6 && e == hipSuccess; ++s) e = dalloc(c, surfs[s], c->plane);
     if (e == hipSuccess) e = dalloc(c, &c->dmean, 3 * c->nlev);
+    if (e == hipSuccess) e = dalloc(c, &c->shift, 3 * c->nlev);
     const size_t B3 = c->plane2 * c->nlev;
     if (e == hipSuccess) e = dalloc(c, &c->u_big, B3);
     if (e == hipSuccess) e = dalloc(c, &c->v_big, B3);
@@ -1123,6 +1177,8 @@ int les_destroy(les_ctx* c) {
     if (c->ev_obk) (void)hipEventDestroy(c->ev_obk);
     if (c->ev_th) (void)hipEventDestroy(c->ev_th);
     if (c->ev_uvw) (void)hipEventDestroy(c->ev_uvw);
+    if (c->ev_xf) (void)hipEventDestroy(c->ev_xf);
+    if (c->ev_yf) (void)hipEventDestroy(c->ev_yf);
     if (c->aux) (void)hipStreamDestroy(c->aux);
     if (c->sums) (void)hipStreamDestroy(c->sums);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1449,15 +1505,18 @@ int les_run(les_ctx* c, int jt0, int nsteps, int* failed_jt) {
     while (done < nsteps) {
         const int chunk = (nsteps - done) < c->cfl_cap ? (nsteps - done) : c->cfl_cap;
         for (int s = 0; s < chunk; ++s) {
-            // check_cfl of newstep (901_debug.f90:85-99), with sgs_stag's u_lag
-            // accumulation in the same pass (u, v, w do not change in between)
+            // check_cfl of newstep (901_debug.f90:85-99), with the vertical
+            // differences and sgs_stag's u_lag accumulation in the same pass
+            // (u, v, w do not change in between)
             const bool lag = c->fuse && !c->sgs_frozen;
             // the sums read u, v, psi_m, sgs_t3 and theta at the wall level,
             // which the CFL pass leaves alone
             obukhov_sums_fork(c, jt0 + done + s);
             c->obk_early = 1;
-            max3_dev(c, c->cfl_dev + s, lag);
+            if (c->fuse) LES_DISPATCH(step_begin_dev, c, c->cfl_dev + s, lag);
+            else max3_dev(c, c->cfl_dev + s);
             c->lag_done = lag;
+            c->ddz_done = c->fuse;
             LES_DISPATCH(step_body, c, jt0 + done + s);
             c->lag_done = 0;
         }

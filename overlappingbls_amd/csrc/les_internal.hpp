@@ -80,6 +80,7 @@ struct les_ctx {
     hipEvent_t ev_fork, ev_join;
     hipEvent_t ev_obk, ev_th;       // obukhov sums done (sums) / plane means of theta done (aux)
     hipEvent_t ev_uvw;              // convec's padded u, v, w done on aux
+    hipEvent_t ev_xf, ev_yf;        // filter_data's x pass done (stream) / y pass done (sums)
     // device fields (FP64), nlev planes each
     double* f3[LES_N_FIELDS3D];
     // work fields in the precision of the current mode (double: f3[id];
@@ -88,6 +89,7 @@ struct les_ctx {
     float* f32buf[LES_N_FIELDS3D];  // FP32 work fields, allocated on the first switch to LES_MIXED
     les::cx<float>* phf;            // FP32 pressure spectrum of the mixed mode
     double* hzm;                    // FP64 plane sums of the z pressure RHS (nlev)
+    double* shift;                  // u, v, w at the first point of each level (3 nlev), pressure shift
     double* lmean;                  // plane means of u and v (2 nlev), mixed-mode lagrange_Sdep
     // time-averaged slices (flow_slice / theta_slice) and their diagnostics
     int st_use, st_c, st_p;
@@ -132,7 +134,8 @@ struct les_ctx {
     int lin_obj;               // objective of the derivative windows (LES_OBJ_*)
     int fuse;                  // fused kernels (LES_FUSE=0 at creation: the separate ones)
     int overlap;               // theta's RHS and update on aux (LES_OVERLAP=0: in order)
-    int lag_done;              // this step's u_lag accumulation already done (k_max3_lag)
+    int lag_done;              // this step's u_lag accumulation already done (k_step_begin)
+    int ddz_done;              // this step's ddz of u, v, w already done (k_step_begin)
     int obk_early;             // this step's obukhov sums already launched on aux (les_run)
     double* tscr[5];           // theta's private scratch while it runs on aux:
                                // work3[0..2], work3[6], big3[3] stand-ins
@@ -297,6 +300,22 @@ bool cross_unpad_x(hipStream_t s, const ConvIn<T>& a, int scalar, T* o0, T* o1, 
 template <typename T>
 bool vort_pad_x(hipStream_t s, const VortIn<T>& g, T* o0, T* o1, T* o2, int nz, int ny, const Twiddle& tin,
                 const Twiddle& tout);
+// The x pass of the pressure's right-hand side with filter_data's x pass on
+// u, v, w (k_lines_rg.hip); lo, hi: the planes divtz(1), divtz(nz) of Hz's
+// ghost levels; shift: a value of u, v, w per level (single-precision
+// spectra: taken off the mean)
+template <typename W>
+struct PressIn {
+    double *u, *v, *w;
+    const W *lo, *hi;
+    cx<W> *hx, *hy, *hz;
+    const double* shift;
+    int ny, nz;
+    double scale, edge_scale;
+};
+bool press_x_available(const Twiddle& tw);
+template <typename W>
+void press_x(hipStream_t s, const PressIn<W>& a, bool filter, const Twiddle& tw);
 // process-wide switch: 0 forces the generic runtime-length kernels
 extern int g_use_ct;
 
@@ -369,15 +388,19 @@ template <typename W> void dpdz_on(les_ctx* c, W* dpdz, const W* p);
 template <typename W> void press_hz_sums_dev(les_ctx* c, double* out, double modi);
 template <typename W> void dpdz_dev(les_ctx* c);
 // RHS assembly + Admas_Bashforth, and RHS -= grad p + project, each one pass
-template <typename W> void rhs_ab2_dev(les_ctx* c, int jt);
+template <typename W> void rhs_ab2_dev(les_ctx* c, int jt);   // also writes c->shift
 template <typename W> void ab2_dev(les_ctx* c);
+// also dp/dz (103_flosol.f90:174-175), formed from p in the same pass
 template <typename W> void gradp_project_dev(les_ctx* c, int jt, bool theta_rows = true);
+void press_modi_dev(les_ctx* c, cx<double>* h, double modi);
 void theta_rows_dev(les_ctx* c);
 template <typename W> void project_dev(les_ctx* c);
-// check_cfl's maxima to out; lag: with this step's u_lag accumulation
-// (lag_accumulate_dev) in the same pass over u, v, w
+// check_cfl's maxima to out
 constexpr int MAX3_BLOCKS = 2048;  // partial maxima per component (c->red + 64)
-void max3_dev(les_ctx* c, double* out, bool lag = false);
+void max3_dev(les_ctx* c, double* out);
+// the same with the step's vertical differences of u, v, w and (lag) its
+// u_lag accumulation in one pass over u, v, w
+template <typename W> void step_begin_dev(les_ctx* c, double* out, bool lag);
 
 // ---- forward step and the linearised step (les_api.hip, les_lin.hip) ---------
 // modi: lbc = 0's surface-temperature term of the bottom row

@@ -507,6 +507,113 @@ __global__ __launch_bounds__((rg_threads<T, N, N, false>())) void kr_x_r2c(Batch
         [&](int rl) { return (row0 + rl < nrows) ? out + (row0 + rl) * ldc : (cx<T>*)nullptr; }, LH, buf, tw, scale);
 }
 
+// The x pass of the pressure solve's right-hand side and of filter_data on
+// the advanced velocity in one kernel: u, v, w (component blockIdx.y) are read
+// once, their row transforms stored as half spectra times a.scale (r2c of
+// press_stag_array's u / dt, 109_press_stag_array.f90:158-199) and, with
+// FILTER, the rows written back without their x Nyquist mode
+// (006_test_filter.f90:82-105).  The projection subtracts a pressure gradient
+// that has no Nyquist modes (in FP64), so filtering before it is filtering
+// after it.
+// Against a prepared right-hand side, its r2c and a filter pass behind the
+// projection this saves nine field passes of 320 in an FP64 step (with the
+// passes merged in k_step_begin and k_gradp_project: a 10-step window at 256^3
+// 105.2 ms against 109.5 ms).
+// Hz's ghost levels take divtz(1) and divtz(nz) (a.lo, a.hi); Hx, Hy have
+// none.  Transformed in FP64 also for single-precision spectra (the rows are
+// FP64 state); there the level's shift is taken off the kx = 0 coefficient
+// before it is rounded, which changes the mean mode only, and that one is
+// solved from FP64 sums.
+template <typename W, int N, bool FILTER>
+__global__ __launch_bounds__((rg_threads<double, N, N, false>())) void kr_x_press(
+    PressIn<W> a, const cx<double>* __restrict__ tw_g) {
+    using T = double;
+    constexpr int NL = rg_lines<T, N, N, false>();
+    constexpr int NTH = rg_threads<T, N, N, false>();
+    constexpr int LS = rg_ls(N);
+    constexpr int SF = rg_nst(N);
+    constexpr int LH = N / 2 + 1;
+    __shared__ cx<T> buf[NL * LS];
+    __shared__ cx<T> tw[N];
+    load_twr(tw, tw_g, N);
+    const int f = blockIdx.y;
+    double* __restrict__ src = f == 0 ? a.u : (f == 1 ? a.v : a.w);
+    cx<W>* __restrict__ out = f == 0 ? a.hx : (f == 1 ? a.hy : a.hz);
+    const int row0 = (int)blockIdx.x * 2 * NL;
+    const int nrows = (a.nz + 1) * a.ny;
+    // ny is even, so the two rows of a line lie on one level
+    auto level = [&](int line) { return (row0 + 2 * line) / a.ny; };
+    auto live = [&](int lev) { return lev >= 1 && lev < a.nz; };   // a level of the field itself
+    __syncthreads();
+    Stage<T, N, 0, -1, NL, NTH, false> f0;
+    f0.load([&](int line, int p) {
+        const int ra = row0 + 2 * line;
+        if (ra >= nrows) return cx<T>{T(0), T(0)};
+        const int lev = ra / a.ny;
+        if (live(lev)) {
+            const double* q = src + (long)ra * N + p;
+            return cx<T>{q[0], q[N]};
+        }
+        if (f < 2) return cx<T>{T(0), T(0)};
+        const W* q = (lev == 0 ? a.lo + (long)ra * N : a.hi + (long)(ra - lev * a.ny) * N) + p;
+        return cx<T>{(T)q[0], (T)q[N]};
+    });
+    f0.compute(tw);
+    f0.template write<LS>(buf);
+    __syncthreads();
+    middle_stages<T, N, -1, NL, NTH, false, LS>(buf, tw);
+    Stage<T, N, SF - 1, -1, NL, NTH, false> fl;
+    fl.template read<LS>(buf);
+    fl.compute(tw);
+    __syncthreads();
+    fl.store([&](int line, int p, cx<T> z) { buf[line * LS + rg_pad(p)] = z; });
+    __syncthreads();
+    for (int e = threadIdx.x; e < 2 * NL * LH; e += NTH) {
+        const int rl = e / LH, k = e - rl * LH;
+        const int row = row0 + rl, lev = row / a.ny;
+        if (row >= nrows || (f < 2 && !live(lev))) continue;
+        cx<T> r = {T(0), T(0)};
+        if (2 * k != N) {
+            const cx<T> zk = buf[(rl >> 1) * LS + rg_pad(k)];
+            const cx<T> zc = buf[(rl >> 1) * LS + rg_pad((N - k) % N)];
+            if ((rl & 1) == 0) r = {(zk.x + zc.x) * T(0.5), (zk.y - zc.y) * T(0.5)};
+            else r = {(zk.y + zc.y) * T(0.5), -(zk.x - zc.x) * T(0.5)};
+            if constexpr (sizeof(W) < sizeof(T)) {
+                if (k == 0 && live(lev)) r.x -= (T)N * a.shift[f * (a.nz + 1) + lev];
+            }
+            const T sc = live(lev) ? a.scale : a.edge_scale;
+            r.x *= sc;
+            r.y *= sc;
+        }
+        out[(long)row * LH + k] = {(W)r.x, (W)r.y};
+    }
+    if constexpr (!FILTER) return;
+    // the Nyquist mode taken off and the inverse transform, from registers
+    Stage<T, N, 0, +1, NL, NTH, false> i0;
+#pragma unroll
+    for (int q = 0; q < decltype(i0)::PB; ++q) {
+        int line, b;
+        if (!decltype(i0)::bf(q, line, b)) continue;
+#pragma unroll
+        for (int r = 0; r < decltype(i0)::R; ++r)
+            i0.v[q][r] = same_len_op<T, N, OP_NYQ>(fl.v[q][r], b + r * decltype(i0)::NB, T(0));
+    }
+    i0.compute(tw);
+    __syncthreads();
+    i0.template write<LS>(buf);
+    __syncthreads();
+    middle_stages<T, N, +1, NL, NTH, false, LS>(buf, tw);
+    Stage<T, N, rg_nst(N) - 1, +1, NL, NTH, false> il;
+    il.template read<LS>(buf);
+    il.compute(tw);
+    il.store([&](int line, int p, cx<T> z) {
+        const int ra = row0 + 2 * line;
+        if (ra >= nrows || !live(level(line))) return;
+        src[(long)ra * N + p] = z.x;
+        src[(long)(ra + 1) * N + p] = z.y;
+    });
+}
+
 // x c2r of ifftn_mpi (FFTW c2r: imaginary parts of the DC and Nyquist
 // coefficients ignored); DERIV applies i kx (kx Nyquist = 0) first.
 template <typename T, int N, int DERIV>
@@ -931,6 +1038,7 @@ struct RgOps {
     void (*c2r)(hipStream_t, const cx<T>*, T*, long, int, int, const Twiddle&, int, double, int);
     void (*spec)(hipStream_t, SpecOp, const Batch<cx<T>, cx<T>>&, int, int, long, const Twiddle&, const double*, int, int,
                  int);
+    void (*press)(hipStream_t, const PressIn<T>&, int, const Twiddle&);
     void (*cross)(hipStream_t, const ConvIn<T>&, int, T*, T*, T*, int, int, const Twiddle&, const Twiddle&);
     void (*vort)(hipStream_t, const VortIn<T>&, T*, T*, T*, int, int, const Twiddle&, const Twiddle&);
     // null where the half length has no two-stage plan
@@ -1032,6 +1140,19 @@ struct RgOpsOf {
             default: spec_o<SP_MULINV>(s, io, np, ncols, ps, tw, G, ld, ldG, mc); break;
         }
     }
+    static void press(hipStream_t s, const PressIn<T>& a, int filter, const Twiddle& tw) {
+        constexpr int NL = rg_lines<double, N, N, false>();
+        constexpr int NTH = rg_threads<double, N, N, false>();
+        const int nrows = (a.nz + 1) * a.ny;
+        const dim3 g((nrows + 2 * NL - 1) / (2 * NL), 3);
+        if constexpr (sizeof(T) == sizeof(double)) {   // the filter comes first in FP64 only
+            if (filter) {
+                hipLaunchKernelGGL((kr_x_press<T, N, true>), g, dim3(NTH), 0, s, a, tw.d);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((kr_x_press<T, N, false>), g, dim3(NTH), 0, s, a, tw.d);
+    }
     template <int NIN, int NOUT, int OP, int NC, typename IN>
     static void fused(hipStream_t s, const IN& a, int comp0, T* o0, T* o1, T* o2, long nrp, int ny_in, long plane_in,
                       int nz, const Twiddle& tin, const Twiddle& tout) {
@@ -1065,7 +1186,7 @@ struct RgOpsOf {
                                    mm, u, cst, twp<T>(tw));
         }
     }
-    static constexpr RgOps<T> table() { return {c2r, spec, cross, vort, lag_has<T>(N) ? lag : nullptr}; }
+    static constexpr RgOps<T> table() { return {c2r, spec, press, cross, vort, lag_has<T>(N) ? lag : nullptr}; }
 };
 
 template <int N>
