@@ -348,6 +348,21 @@ void wallstress(les_ctx* c, int top) {
     wallstress_dev<W>(c, top, w, w + c->plane);
 }
 
+// The filtered fields of lagrange_Sdep are stored only where no contraction
+// kernel takes them as they are transformed back (line lengths without one,
+// LES_FUSE=0): 42 fields, a third of a context's memory, allocated on the
+// first such update.
+bool lag_filtered_buf(les_ctx* c) {
+    if (!c->lag_filt) {
+        const hipError_t e = dalloc(c, &c->lag_filt, 2 * 21 * (size_t)c->nz * c->plane);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            les_note(c, e);
+        }
+    }
+    return c->lag_filt != nullptr;
+}
+
 template <typename W>
 void lagrange(les_ctx* c, int jt) {
     const les_params& P = c->prm;
@@ -355,8 +370,6 @@ void lagrange(les_ctx* c, int jt) {
     const long np21 = 21L * nz;  // planes
     interpolag_dev<W>(c);
     W* raw = scr<W>(c->lag_buf);
-    W* b2 = raw + (size_t)np21 * c->plane;
-    W* b4 = b2 + (size_t)np21 * c->plane;
     // Spectra pruned to the filters' support: kc columns per row, rows
     // min(y, ny - y) < mc.  Modes outside it are zero after either filter,
     // so they are neither stored nor transformed back.
@@ -384,7 +397,9 @@ void lagrange(les_ctx* c, int jt) {
         lag_contract_x<W>(c->stream, 2, spt, kc, kc, nz, c->ny, lmb, mmb, u, cst, c->tw_x)) {
         yline_spec<W>(c->stream, spf, spt, (int)np21, kc4, psp, c->tw_y, SP_MULINV, c->Gtest2, kc, c->lhx, mc);
         lag_contract_x<W>(c->stream, 4, spt, kc, kc4, nz, c->ny, lmb, mmb, u, cst, c->tw_x);
-    } else {
+    } else if (lag_filtered_buf(c)) {
+        W* b2 = scr<W>(c->lag_filt);
+        W* b4 = b2 + (size_t)np21 * c->plane;
         x_c2r<W>(c->stream, spt, b2, np21 * c->ny, kc, c->nx, c->tw_x, 0, 0.0, kc);
         yline_spec<W>(c->stream, spf, spt, (int)np21, kc4, psp, c->tw_y, SP_MULINV, c->Gtest2, kc, c->lhx, mc);
         x_c2r<W>(c->stream, spt, b4, np21 * c->ny, kc, c->nx, c->tw_x, 0, 0.0, kc4);
@@ -1107,9 +1122,7 @@ int les_create(const les_params* prm, les_ctx** out) {
     if (e == hipSuccess) e = dalloc(c, &c->tscr[3], 3 * ((F3 * 3) / 2) + c->plane2);
     if (e == hipSuccess) e = dalloc(c, &c->tscr[4], B3);
     for (int i = 0; i < 4 && e == hipSuccess; ++i) e = dalloc(c, &c->spec3[i], c->ns * c->nlev);
-    const size_t np21 = (size_t)21 * c->nz;
-    if (e == hipSuccess) e = dalloc(c, &c->lag_buf, 3 * np21 * c->plane);
-    if (e == hipSuccess) e = dalloc(c, &c->lag_spec, 2 * np21 * c->ns);
+    if (e == hipSuccess) e = dalloc(c, &c->lag_buf, (size_t)21 * c->nz * c->plane);
     for (int i = 0; i < 4 && e == hipSuccess; ++i) e = dalloc(c, &c->fold[i], F3);
     if (e == hipSuccess) e = dalloc(c, &c->scal, 64);
     if (e == hipSuccess) e = dalloc(c, &c->red, 64 + 3 * MAX3_BLOCKS + c->nlev);
@@ -1129,6 +1142,11 @@ int les_create(const les_params* prm, les_ctx** out) {
         init_spectral(c) != hipSuccess) {
         les_destroy(c);
         return LES_E_HIP;
+    }
+    // raw and filtered spectra of lagrange_Sdep, pruned to the filters' columns
+    if (dalloc(c, &c->lag_spec, 2 * (size_t)21 * c->nz * c->lag_kc * c->ny) != hipSuccess) {
+        les_destroy(c);
+        return LES_E_NOMEM;
     }
     for (int f = 0; f < LES_N_FIELDS3D; ++f) les_note(c, hipMemsetAsync(c->f3[f], 0, F3 * 8, c->stream));
     for (int f = 0; f < LES_N_FIELDS3D; ++f) c->wk[f] = is_work_field(f) ? (void*)c->f3[f] : nullptr;
