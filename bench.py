@@ -290,7 +290,7 @@ def adjoint_leg(workload="sbl128", nsteps=20, k_ckpt=5, obj_steps=5, ndir=8, eps
 # the last template argument: 0 derivative, 1 Nyquist filter, 2 pad, 3 unpad.
 _LINE_OPS = {"0": "deriv", "1": "filter", "2": "pad", "3": "unpad"}
 _POINT_FAMILIES = [
-    (("k_obukhov_sums", "k_level_means_seq"), "plane_sums"),
+    (("k_obukhov_sums", "k_level_means_"), "plane_sums"),
     (("k_rhs_ab2",), "rhs_ab2"),
     (("k_gradp_project", "k_project_bc"), "gradp_project"),
     (("k_strain_stress", "k_strain<", "k_stress<"), "sgs_stress"),
@@ -307,6 +307,7 @@ _POINT_FAMILIES = [
     (("kr_x_c2r", "k_x_c2r"), "x_c2r"),
     (("kr_yspec", "k_yline_spec"), "yline.spec"),
     (("k_vort<",), "vort_pad_x"),
+    (("kr_cross_x",), "cross_unpad_x"),
 ]
 # the first kernel of every step: obukhov's plane sums, which les_run launches
 # before the CFL pass, or the CFL pass where a step has no such sums
@@ -322,10 +323,7 @@ def kernel_family(name: str) -> str:
     if m:
         return f"{m.group(1)}line.{_LINE_OPS[m.group(2)]}"
     if "kr_fused_x" in name:
-        if "VortIn" in name:
-            return "vort_pad_x"
-        m = re.search(r"kr_fused_x<[^,]+, \d+, \d+, \d+, (\d+),", name)
-        return "scalar_unpad_x" if (m and m.group(1) == "1") else "cross_unpad_x"
+        return "vort_pad_x" if "VortIn" in name else "scalar_unpad_x"
     for keys, fam in _POINT_FAMILIES:
         if any(k in name for k in keys):
             return fam

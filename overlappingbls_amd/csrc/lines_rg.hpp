@@ -782,38 +782,21 @@ inline long xcd_blocks(long ngroups) {
 // rounds it), then runs the x pass from LDS: the product or vorticity field
 // is never written to and re-read from memory.
 //
-// A block takes one component (consecutive blocks of an XCD take the
-// components of the same rows, so the shared inputs are re-read from cache)
+// A block takes one component (of the vorticity: three that share no input)
 // and one group of FusedWork: line l is the row pair of its column on level
-// k0 + 1 + l.  The evaluation is branch
-// free (every input loaded, the wall-level formula chosen by a select), so
-// the loads of all of a thread's elements can be in flight together.
+// k0 + 1 + l.  The evaluation is branch free (every input loaded, the
+// wall-level formula chosen by a select), so the loads of all of a thread's
+// elements can be in flight together.  The cross product, whose components
+// share their inputs, has a kernel of its own (kr_cross_x).
 template <typename T, int COMP>
 __device__ __forceinline__ double fused_value(const ConvIn<T>& a, int k, long i, long P2, int) {
-    if constexpr (COMP == 3) {  // scalar advection
-        const T ub = a.ub[i], vb = a.vb[i], wb = a.wb[i], wp = a.wb[i + P2];
-        const T sx = a.b1[i], sy = a.b2[i], sz = a.b3[i], szp = a.b3[i + P2];
-        const double ust = a.ust[k], vst = a.vst[k];
-        const double w1 = (ub + ust) * sx + (vb + vst) * sy + (0.5 * wp) * szp;
-        const double wg = (ub + ust) * sx + (vb + vst) * sy + ((double)wb * sz + (double)wp * szp) / 2.0;
-        return (k == 1) ? w1 : wg;
-    } else if constexpr (COMP == 0) {
-        const T vb = a.vb[i], b3 = a.b3[i], wp = a.wb[i + P2], b2p = a.b2[i + P2], wb = a.wb[i], b2 = a.b2[i];
-        const double vst = a.vst[k];
-        const double w1 = (vb + vst) * (-b3) + 0.5 * wp * b2p;
-        const double wg = (vb + vst) * (-b3) + 0.5 * (wp * (b2p) + wb * (b2));
-        return (k == 1) ? w1 : wg;
-    } else if constexpr (COMP == 1) {
-        const T ub = a.ub[i], b3 = a.b3[i], wp = a.wb[i + P2], b1p = a.b1[i + P2], wb = a.wb[i], b1 = a.b1[i];
-        const double ust = a.ust[k];
-        const double w1 = (ub + ust) * (b3) + 0.5 * wp * (-b1p);
-        const double wg = (ub + ust) * (b3) + 0.5 * (wp * (-b1p) + wb * (-b1));
-        return (k == 1) ? w1 : wg;
-    } else {
-        const T ub = a.ub[i], um = a.ub[i - P2], b2 = a.b2[i], vb = a.vb[i], vm = a.vb[i - P2], b1 = a.b1[i];
-        const double wg = 0.5 * ((ub + um + a.ust[k] + a.ust[k - 1]) * (-b2) + (vb + vm + a.vst[k] + a.vst[k - 1]) * (b1));
-        return (k == 1) ? 0.0 : wg;
-    }
+    // scalar advection
+    const T ub = a.ub[i], vb = a.vb[i], wb = a.wb[i], wp = a.wb[i + P2];
+    const T sx = a.b1[i], sy = a.b2[i], sz = a.b3[i], szp = a.b3[i + P2];
+    const double ust = a.ust[k], vst = a.vst[k];
+    const double w1 = (ub + ust) * sx + (vb + vst) * sy + (0.5 * wp) * szp;
+    const double wg = (ub + ust) * sx + (vb + vst) * sy + ((double)wb * sz + (double)wp * szp) / 2.0;
+    return (k == 1) ? w1 : wg;
 }
 template <typename T, int COMP>
 __device__ __forceinline__ double fused_value(const VortIn<T>& g, int k, long i, long P, int nz) {
@@ -879,15 +862,33 @@ struct FusedWork {
     }
 };
 
-// NC components per row pair; comp0 is the first component's index (3 for
-// the scalar advection).  ny_in rows per level, plane_in values per plane;
-// nrp = levels * ny_in / 2 row pairs.
+// Lines and threads of a block, measured at 256 <-> 384, 256 levels: the
+// vorticity's pads (global twiddles, so its LDS is the lines alone) take half
+// the lines of an ordinary x pass, more blocks a CU (FP64 431 -> 365 us), in
+// FP32 with twice the threads the transform has butterflies for, for the
+// loads' sake (249 -> 222 us; slower in FP64); a quarter of the lines: 698 and
+// 326 us.  The advection's unpads take the ordinary lines and twice the
+// threads (FP64 450 -> 443, FP32 235 -> 226 us).
+template <typename T, int NIN, int NOUT>
+constexpr int fused_lines() {
+    constexpr int mb = cmax(rg_maxbf(NIN), rg_maxbf(NOUT));
+    return NIN < NOUT ? cmax(1, 64 / mb) : rg_lines<T, NIN, NOUT, false>();
+}
+template <typename T, int NIN, int NOUT>
+constexpr int fused_threads() {
+    constexpr int mb = cmax(rg_maxbf(NIN), rg_maxbf(NOUT));
+    return round64(fused_lines<T, NIN, NOUT>() * mb) * (NIN < NOUT && sizeof(T) == 8 ? 1 : 2);
+}
+
+// NC components per row pair (1: the scalar advection, 3: the vorticity).
+// ny_in rows per level, plane_in values per plane; nrp = levels * ny_in / 2
+// row pairs.
 template <typename T, int NIN, int NOUT, int OP, int NC, typename IN>
-__global__ __launch_bounds__((rg_threads<T, NIN, NOUT, false>())) void kr_fused_x(
-    IN a, int comp0, T* o0, T* o1, T* o2, long nrp, int ny_in, long plane_in, int nz,
+__global__ __launch_bounds__((fused_threads<T, NIN, NOUT>())) void kr_fused_x(
+    IN a, T* o0, T* o1, T* o2, long nrp, int ny_in, long plane_in, int nz,
     const cx<T>* __restrict__ twin_g, const cx<T>* __restrict__ twout_g) {
-    constexpr int NL = rg_lines<T, NIN, NOUT, false>();
-    constexpr int NTH = rg_threads<T, NIN, NOUT, false>();
+    constexpr int NL = fused_lines<T, NIN, NOUT>();
+    constexpr int NTH = fused_threads<T, NIN, NOUT>();
     constexpr int LS = rg_ls(cmax(NIN, NOUT));
     constexpr bool TWG = tw_global<NIN, NOUT>();
     __shared__ cx<T> buf[NL * LS];
@@ -908,11 +909,11 @@ __global__ __launch_bounds__((rg_threads<T, NIN, NOUT, false>())) void kr_fused_
     int col, k0;
     wk.item(rg, col, k0);
     if (col >= wk.ycols) return;  // whole workgroup: a padding column
-    const int comp = comp0 + cb;
-    if (comp == 0) fused_inputs<T, NIN, NL, NTH, LS, 0>(a, buf, k0, col, wk.nlz, plane_in, nz);
-    else if (comp == 1) fused_inputs<T, NIN, NL, NTH, LS, 1>(a, buf, k0, col, wk.nlz, plane_in, nz);
-    else if (comp == 2) fused_inputs<T, NIN, NL, NTH, LS, 2>(a, buf, k0, col, wk.nlz, plane_in, nz);
-    else fused_inputs<T, NIN, NL, NTH, LS, 3>(a, buf, k0, col, wk.nlz, plane_in, nz);
+    if (cb == 0) fused_inputs<T, NIN, NL, NTH, LS, 0>(a, buf, k0, col, wk.nlz, plane_in, nz);
+    if constexpr (NC == 3) {
+        if (cb == 1) fused_inputs<T, NIN, NL, NTH, LS, 1>(a, buf, k0, col, wk.nlz, plane_in, nz);
+        else if (cb == 2) fused_inputs<T, NIN, NL, NTH, LS, 2>(a, buf, k0, col, wk.nlz, plane_in, nz);
+    }
     __syncthreads();
     T* o = (cb == 0) ? o0 : ((cb == 1) ? o1 : o2);
     auto ld = [&](int line, int p) { return buf[line * LS + rg_pad(p)]; };
@@ -924,6 +925,105 @@ __global__ __launch_bounds__((rg_threads<T, NIN, NOUT, false>())) void kr_fused_
         o[(r + 1) * NOUT + p] = z.y;
     };
     line_pipeline<T, NIN, NOUT, OP, NL, NTH, false, true>(ld, st, buf, twi, twop, T(0));
+}
+
+// ---- cross product and the x pass of its unpads -------------------------------
+// (108_convec.f90:103-202).  A block takes one row pair on NLV consecutive
+// levels, all three components: a thread reads its positions of u, v, w and
+// the vorticity on the levels and their neighbours once, all loads in flight
+// together, and forms the 3 NLV lines in LDS.  A block per component (the
+// form of kr_fused_x) reads every field two or three times from cache and, at
+// 3.2 TB/s, was bound by those reads' latency at six waves a CU: 256 x 256 x
+// 256 levels, 777 -> 526 us in FP64 (4.6 TB/s) and 363 -> 275 us in FP32.
+// Three levels: 559 / 287 us with two, 581 with two and the store's pointers
+// in memory, 718 / 488 with four, 666 with one.  Twiddle tables in LDS (579 /
+// 310 us through the vector cache).
+// NLV: as many of three levels as leave two workgroups on a CU and 512 threads.
+template <typename T, int NIN, int NOUT>
+struct CrossShape {
+    static constexpr int mb = cmax(rg_maxbf(NIN), rg_maxbf(NOUT));
+    static constexpr int lds(int nl) { return (3 * nl * rg_ls(NIN) + NIN + NOUT) * (int)sizeof(cx<T>); }
+    static constexpr int levels() {
+        int nl = 3;
+        while (nl > 1 && (3 * nl * mb > 512 || lds(nl) > 81920)) --nl;
+        return nl;
+    }
+    static constexpr int NLV = levels();
+    static constexpr int NTH = round64(3 * NLV * mb);
+    static_assert(lds(NLV) <= 81920, "two workgroups a CU");
+};
+template <typename T, int NIN, int NOUT>
+__global__ __launch_bounds__((CrossShape<T, NIN, NOUT>::NTH)) void kr_cross_x(
+    ConvIn<T> a, T* o0, T* o1, T* o2, long nrp, int ny_in, long plane_in, const cx<T>* __restrict__ twin_g,
+    const cx<T>* __restrict__ twout_g) {
+    using S = CrossShape<T, NIN, NOUT>;
+    constexpr int NLV = S::NLV, NTH = S::NTH, LS = rg_ls(NIN), PER = (NIN + NTH - 1) / NTH;
+    __shared__ cx<T> buf[3 * NLV * LS];
+    __shared__ cx<T> twl[NIN], twl_o[NOUT];
+    load_twr(twl, twin_g, NIN);
+    load_twr(twl_o, twout_g, NOUT);
+    long rg;
+    int cb;
+    xcd_item<1>(rg, cb);
+    const FusedWork<NLV> wk(nrp, ny_in);
+    int col, k0;
+    wk.item(rg, col, k0);
+    if (col >= wk.ycols) return;  // whole workgroup: a padding column
+    // lines: component c of level 1 + k0 + l is line c NLV + l
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int p = (int)threadIdx.x + j * NTH;
+        if (NIN % NTH != 0 && p >= NIN) break;
+        const long i0 = (long)(2 * col) * NIN + p;
+        T u[2][NLV + 1], v[2][NLV + 1], w[2][NLV + 1], b1[2][NLV + 1], b2[2][NLV + 1], b3[2][NLV];
+#pragma unroll
+        for (int l = 0; l <= NLV; ++l) {
+            // levels past the last read it and are not stored
+            const long iu = i0 + (long)min(k0 + l, wk.nlz) * plane_in;          // u, v from level k0
+            const long iw = i0 + (long)min(k0 + l + 1, wk.nlz + 1) * plane_in;  // the others from k0 + 1
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                u[r][l] = a.ub[iu + r * NIN];
+                v[r][l] = a.vb[iu + r * NIN];
+                w[r][l] = a.wb[iw + r * NIN];
+                b1[r][l] = a.b1[iw + r * NIN];
+                b2[r][l] = a.b2[iw + r * NIN];
+                if (l < NLV) b3[r][l] = a.b3[iw + r * NIN];
+            }
+        }
+#pragma unroll
+        for (int l = 0; l < NLV; ++l) {
+            const int k = min(1 + k0 + l, wk.nlz);
+            const double ust = a.ust[k], vst = a.vst[k], usm = a.ust[k - 1], vsm = a.vst[k - 1];
+            T x[2], y[2], z[2];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const T ub = u[r][l + 1], um = u[r][l], vb = v[r][l + 1], vm = v[r][l], wb = w[r][l], wp = w[r][l + 1];
+                const T b1k = b1[r][l], b1p = b1[r][l + 1], b2k = b2[r][l], b2p = b2[r][l + 1], b3k = b3[r][l];
+                const double x1 = (vb + vst) * (-b3k) + 0.5 * wp * b2p;
+                const double xg = (vb + vst) * (-b3k) + 0.5 * (wp * (b2p) + wb * (b2k));
+                x[r] = (T)((k == 1) ? x1 : xg);
+                const double y1 = (ub + ust) * (b3k) + 0.5 * wp * (-b1p);
+                const double yg = (ub + ust) * (b3k) + 0.5 * (wp * (-b1p) + wb * (-b1k));
+                y[r] = (T)((k == 1) ? y1 : yg);
+                const double zg = 0.5 * ((ub + um + ust + usm) * (-b2k) + (vb + vm + vst + vsm) * (b1k));
+                z[r] = (T)((k == 1) ? 0.0 : zg);
+            }
+            buf[l * LS + rg_pad(p)] = {x[0], x[1]};
+            buf[(NLV + l) * LS + rg_pad(p)] = {y[0], y[1]};
+            buf[(2 * NLV + l) * LS + rg_pad(p)] = {z[0], z[1]};
+        }
+    }
+    __syncthreads();
+    auto ld = [&](int line, int p) { return buf[line * LS + rg_pad(p)]; };
+    auto st = [=](int line, int p, cx<T> z) {   // by value: the choice of pointer stays in registers
+        const int c = line / NLV, kl = k0 + line - c * NLV;
+        if (kl >= wk.nlz) return;
+        T* o = (c == 0 ? o0 : (c == 1 ? o1 : o2)) + ((long)kl * (2 * wk.ycols) + 2 * col) * NOUT + p;
+        o[0] = z.x;
+        o[NOUT] = z.y;
+    };
+    line_pipeline<T, NIN, NOUT, OP_UNPAD, 3 * NLV, NTH, false, true>(ld, st, buf, twl, twl_o, T(0));
 }
 
 // ---- lagrange_Sdep: filtered fields contracted as they are transformed back ----
@@ -1154,24 +1254,30 @@ struct RgOpsOf {
         hipLaunchKernelGGL((kr_x_press<T, N, false>), g, dim3(NTH), 0, s, a, tw.d);
     }
     template <int NIN, int NOUT, int OP, int NC, typename IN>
-    static void fused(hipStream_t s, const IN& a, int comp0, T* o0, T* o1, T* o2, long nrp, int ny_in, long plane_in,
+    static void fused(hipStream_t s, const IN& a, T* o0, T* o1, T* o2, long nrp, int ny_in, long plane_in,
                       int nz, const Twiddle& tin, const Twiddle& tout) {
-        constexpr int NL = rg_lines<T, NIN, NOUT, false>();
-        constexpr int NTH = rg_threads<T, NIN, NOUT, false>();
+        constexpr int NL = fused_lines<T, NIN, NOUT>();
+        constexpr int NTH = fused_threads<T, NIN, NOUT>();
         const long nb = xcd_blocks<NC>(FusedWork<NL>(nrp, ny_in).groups());
-        hipLaunchKernelGGL((kr_fused_x<T, NIN, NOUT, OP, NC, IN>), dim3((unsigned)nb), dim3(NTH), 0, s, a, comp0, o0,
+        hipLaunchKernelGGL((kr_fused_x<T, NIN, NOUT, OP, NC, IN>), dim3((unsigned)nb), dim3(NTH), 0, s, a, o0,
                            o1, o2, nrp, ny_in, plane_in, nz, twp<T>(tin), twp<T>(tout));
     }
     static void cross(hipStream_t s, const ConvIn<T>& a, int scalar, T* o0, T* o1, T* o2, int nz, int ny2,
                       const Twiddle& tin, const Twiddle& tout) {
         constexpr int M = 3 * N / 2;
         const long plane2 = (long)M * ny2, nrp = (long)(nz - 1) * ny2 / 2;
-        if (scalar) fused<M, N, OP_UNPAD, 1>(s, a, 3, o0, o1, o2, nrp, ny2, plane2, nz, tin, tout);
-        else fused<M, N, OP_UNPAD, 3>(s, a, 0, o0, o1, o2, nrp, ny2, plane2, nz, tin, tout);
+        if (scalar) {
+            fused<M, N, OP_UNPAD, 1>(s, a, o0, o1, o2, nrp, ny2, plane2, nz, tin, tout);
+        } else {
+            using S = CrossShape<T, M, N>;
+            const long nb = xcd_blocks<1>(FusedWork<S::NLV>(nrp, ny2).groups());
+            hipLaunchKernelGGL((kr_cross_x<T, M, N>), dim3((unsigned)nb), dim3(S::NTH), 0, s, a, o0, o1, o2, nrp, ny2,
+                               plane2, twp<T>(tin), twp<T>(tout));
+        }
     }
     static void vort(hipStream_t s, const VortIn<T>& g, T* o0, T* o1, T* o2, int nz, int ny, const Twiddle& tin,
                      const Twiddle& tout) {
-        fused<N, 3 * N / 2, OP_PAD, 3>(s, g, 0, o0, o1, o2, (long)nz * ny / 2, ny, (long)N * ny, nz, tin, tout);
+        fused<N, 3 * N / 2, OP_PAD, 3>(s, g, o0, o1, o2, (long)nz * ny / 2, ny, (long)N * ny, nz, tin, tout);
     }
     static void lag(hipStream_t s, int scale, const cx<T>* spt, int ldc, int kst, int nz, int ny, double* lm,
                     double* mm, const LagUpdate& u, double cst, const Twiddle& tw) {
