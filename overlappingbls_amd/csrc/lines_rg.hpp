@@ -936,21 +936,27 @@ __global__ __launch_bounds__((fused_threads<T, NIN, NOUT>())) void kr_fused_x(
 // 3.2 TB/s, was bound by those reads' latency at six waves a CU: 256 x 256 x
 // 256 levels, 777 -> 526 us in FP64 (4.6 TB/s) and 363 -> 275 us in FP32.
 // Three levels: 559 / 287 us with two, 581 with two and the store's pointers
-// in memory, 718 / 488 with four, 666 with one.  Twiddle tables in LDS (579 /
-// 310 us through the vector cache).
-// NLV: as many of three levels as leave two workgroups on a CU and 512 threads.
+// in memory, 718 / 488 with four, 666 with one.
+// NLV: as many of three levels as leave two workgroups on a CU and 512 threads,
+// with the twiddle tables in LDS (three levels with them read through the
+// vector cache: 579 / 310 us), unless that leaves one level: 768-point rows in
+// FP64 take two levels and the tables from the cache (512 x 512 x 65 levels:
+// 757 us; one level and tables in LDS 995, a block per component 937).
 template <typename T, int NIN, int NOUT>
 struct CrossShape {
     static constexpr int mb = cmax(rg_maxbf(NIN), rg_maxbf(NOUT));
-    static constexpr int lds(int nl) { return (3 * nl * rg_ls(NIN) + NIN + NOUT) * (int)sizeof(cx<T>); }
-    static constexpr int levels() {
+    static constexpr int lds(int nl, bool tables) {
+        return (3 * nl * rg_ls(NIN) + (tables ? NIN + NOUT : 0)) * (int)sizeof(cx<T>);
+    }
+    static constexpr int levels(bool tables) {
         int nl = 3;
-        while (nl > 1 && (3 * nl * mb > 512 || lds(nl) > 81920)) --nl;
+        while (nl > 1 && (3 * nl * mb > 512 || lds(nl, tables) > 81920)) --nl;
         return nl;
     }
-    static constexpr int NLV = levels();
+    static constexpr bool TWL = levels(true) > 1;
+    static constexpr int NLV = levels(TWL);
     static constexpr int NTH = round64(3 * NLV * mb);
-    static_assert(lds(NLV) <= 81920, "two workgroups a CU");
+    static_assert(lds(NLV, TWL) <= 81920, "two workgroups a CU");
 };
 template <typename T, int NIN, int NOUT>
 __global__ __launch_bounds__((CrossShape<T, NIN, NOUT>::NTH)) void kr_cross_x(
@@ -959,9 +965,14 @@ __global__ __launch_bounds__((CrossShape<T, NIN, NOUT>::NTH)) void kr_cross_x(
     using S = CrossShape<T, NIN, NOUT>;
     constexpr int NLV = S::NLV, NTH = S::NTH, LS = rg_ls(NIN), PER = (NIN + NTH - 1) / NTH;
     __shared__ cx<T> buf[3 * NLV * LS];
-    __shared__ cx<T> twl[NIN], twl_o[NOUT];
-    load_twr(twl, twin_g, NIN);
-    load_twr(twl_o, twout_g, NOUT);
+    __shared__ cx<T> twl[S::TWL ? NIN : 1], twl_o[S::TWL ? NOUT : 1];
+    const cx<T>*twi = twin_g, *twop = twout_g;
+    if constexpr (S::TWL) {
+        load_twr(twl, twin_g, NIN);
+        load_twr(twl_o, twout_g, NOUT);
+        twi = twl;
+        twop = twl_o;
+    }
     long rg;
     int cb;
     xcd_item<1>(rg, cb);
@@ -1023,7 +1034,7 @@ __global__ __launch_bounds__((CrossShape<T, NIN, NOUT>::NTH)) void kr_cross_x(
         o[0] = z.x;
         o[NOUT] = z.y;
     };
-    line_pipeline<T, NIN, NOUT, OP_UNPAD, 3 * NLV, NTH, false, true>(ld, st, buf, twl, twl_o, T(0));
+    line_pipeline<T, NIN, NOUT, OP_UNPAD, 3 * NLV, NTH, false, true>(ld, st, buf, twi, twop, T(0));
 }
 
 // ---- lagrange_Sdep: filtered fields contracted as they are transformed back ----
