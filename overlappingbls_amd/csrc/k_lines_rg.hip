@@ -129,6 +129,10 @@ bool vort_pad_x(hipStream_t s, const VortIn<T>& g, T* o0, T* o1, T* o2, int nz, 
     rg_ops<T>(t).vort(s, g, o0, o1, o2, nz, ny, tin, tout);
     return true;
 }
+bool lag_contract_available(const Twiddle& tw) {
+    const RgTable* t = rg_table(tw.n);
+    return t && rg_ops<double>(t).lag && rg_ops<float>(t).lag;
+}
 template <typename T>
 bool lag_contract_x(hipStream_t s, int scale, const cx<T>* spt, int ldc, int kst, int nz, int ny, double* lm,
                     double* mm, const LagUpdate& u, double cst, const Twiddle& tw) {

@@ -348,21 +348,6 @@ void wallstress(les_ctx* c, int top) {
     wallstress_dev<W>(c, top, w, w + c->plane);
 }
 
-// The filtered fields of lagrange_Sdep are stored only where no contraction
-// kernel takes them as they are transformed back (line lengths without one,
-// LES_FUSE=0): 42 fields, a third of a context's memory, allocated on the
-// first such update.
-bool lag_filtered_buf(les_ctx* c) {
-    if (!c->lag_filt) {
-        const hipError_t e = dalloc(c, &c->lag_filt, 2 * 21 * (size_t)c->nz * c->plane);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            les_note(c, e);
-        }
-    }
-    return c->lag_filt != nullptr;
-}
-
 template <typename W>
 void lagrange(les_ctx* c, int jt) {
     const les_params& P = c->prm;
@@ -393,11 +378,11 @@ void lagrange(les_ctx* c, int jt) {
     double* lmb = c->lag_buf;
     double* mmb = c->lag_buf + c->plane * c->nlev;
     const double cst = 2.0 * (delta * delta);
-    if (c->fuse && g_use_ct &&
+    if ((!c->lag_filt || (c->fuse && g_use_ct)) &&
         lag_contract_x<W>(c->stream, 2, spt, kc, kc, nz, c->ny, lmb, mmb, u, cst, c->tw_x)) {
         yline_spec<W>(c->stream, spf, spt, (int)np21, kc4, psp, c->tw_y, SP_MULINV, c->Gtest2, kc, c->lhx, mc);
         lag_contract_x<W>(c->stream, 4, spt, kc, kc4, nz, c->ny, lmb, mmb, u, cst, c->tw_x);
-    } else if (lag_filtered_buf(c)) {
+    } else {
         W* b2 = scr<W>(c->lag_filt);
         W* b4 = b2 + (size_t)np21 * c->plane;
         x_c2r<W>(c->stream, spt, b2, np21 * c->ny, kc, c->nx, c->tw_x, 0, 0.0, kc);
@@ -1143,8 +1128,15 @@ int les_create(const les_params* prm, les_ctx** out) {
         les_destroy(c);
         return LES_E_HIP;
     }
-    // raw and filtered spectra of lagrange_Sdep, pruned to the filters' columns
-    if (dalloc(c, &c->lag_spec, 2 * (size_t)21 * c->nz * c->lag_kc * c->ny) != hipSuccess) {
+    // raw and filtered spectra of lagrange_Sdep, pruned to the filters' columns;
+    // its filtered fields (42, a third of a context's memory) only where no
+    // contraction kernel takes them as they are transformed back: row lengths
+    // without one, LES_FUSE=0, the runtime-length kernels.  A context without
+    // them keeps the contraction kernels if that process-wide switch is set later.
+    const bool contract = c->fuse && g_use_ct && lag_contract_available(c->tw_x);
+    const size_t np21 = (size_t)21 * c->nz;
+    if (dalloc(c, &c->lag_spec, 2 * np21 * c->lag_kc * c->ny) != hipSuccess ||
+        (!contract && dalloc(c, &c->lag_filt, 2 * np21 * c->plane) != hipSuccess)) {
         les_destroy(c);
         return LES_E_NOMEM;
     }

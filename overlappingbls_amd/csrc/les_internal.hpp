@@ -122,7 +122,7 @@ struct les_ctx {
     double* th1_copy;          // theta(1) for the obukhov sums (one plane)
     les::cx<double>* spec3[4]; // half-spectrum fields (nlev planes of ns): Hx, Hy, Hz, p_hat
     double* lag_buf;           // lagrange_Sdep: 21 fields
-    double* lag_filt;          // their 2 delta and 4 delta filtered forms, or null (lag_filtered_buf)
+    double* lag_filt;          // their 2 delta and 4 delta filtered forms, or null (contraction kernels)
     les::cx<double>* lag_spec; // 2 x 21 pruned spectra
     double* fold[4];           // interpolag copies of F_*
     double* scal;              // device scalars

@@ -74,6 +74,7 @@ __device__ __forceinline__ void lag_update(const LagUpdate& u, long i, int k, do
 // back and contracted in one pass (k_lines_rg.hip): scale 2 writes L M and
 // M M to lm, mm; scale 4 reads them and applies lag_update.  False when the
 // line length has no kernel (the caller then transforms and contracts apart).
+bool lag_contract_available(const Twiddle& tw);   // in both precisions
 template <typename T>
 bool lag_contract_x(hipStream_t s, int scale, const cx<T>* spt, int ldc, int kst, int nz, int ny, double* lm,
                     double* mm, const LagUpdate& u, double cst, const Twiddle& tw);

@@ -1,0 +1,76 @@
+"""The library's host code without a GPU: tests/cpp/fake_hip.cpp stands in for
+the HIP runtime in a child process (kernels are not run), so that memory that
+runs out, a launch that fails and the stream each kernel goes to can be
+checked on the CPU."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+from overlappingbls_amd import build, lib
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PREAMBLE = """
+import ctypes as C, dataclasses, sys
+import numpy as np
+fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+for f in ("fake_nmalloc", "fake_held", "fake_nlaunch", "fake_stream"):
+    getattr(fake, f).restype = C.c_long
+fake.fake_kernel.restype = C.c_char_p
+fake.fake_kernel.argtypes = fake.fake_stream.argtypes = fake.fake_budget.argtypes = [C.c_long]
+from overlappingbls_amd import config, lib
+from overlappingbls_amd.abi import LES_E_HIP, LES_E_NOMEM, LES_MIXED, LES_OK, LesError
+
+def grid(nx, ny, nzt=6, **kw):
+    return dataclasses.replace(config.workload("tiny_ragged"), nxt=nx, nyt=ny, nzt=nzt, **kw).params()
+
+def launches():
+    return [(fake.fake_kernel(i).decode(), fake.fake_stream(i)) for i in range(fake.fake_nlaunch())]
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    gxx, rocm = shutil.which("g++"), os.path.dirname(os.path.dirname(os.path.realpath(build.HIPCC)))
+    if gxx is None:
+        pytest.skip("no g++")
+    if not os.path.exists(lib.LIB):
+        build.build()
+    so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    subprocess.run([gxx, "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I",
+                    os.path.join(rocm, "include"), "-o", so, os.path.join(ROOT, "tests", "cpp", "fake_hip.cpp")],
+                   check=True)
+
+    def child(code, **env):
+        r = subprocess.run([sys.executable, "-c", PREAMBLE + code, so], cwd=ROOT, env={**os.environ, **env},
+                           capture_output=True, text=True)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return child
+
+
+# rows of 24 and 324 values have no contraction kernel, rows of 32 have one
+@pytest.mark.parametrize("nx,fuse", [(24, "1"), (324, "1"), (32, "0"), (32, "1")])
+def test_memory_is_taken_by_create(nx, fuse, fake):
+    """All device memory of a step, dynamic SGS updates among them, belongs to
+    les_create: none is allocated later, a shortage is refused there with
+    LES_E_NOMEM and everything is given back."""
+    fake(f"""
+g = lib.create(grid({nx}, 12))
+n, held = fake.fake_nmalloc(), fake.fake_held()
+g.run(1, 4)
+assert fake.fake_nmalloc() == n, "allocated in a step"
+assert any("lagrange" in k or "lag_" in k for k, s in launches())
+g.close()
+assert fake.fake_held() == 0
+fake.fake_budget(held - 1)
+try:
+    lib.create(grid({nx}, 12))
+except LesError as e:
+    assert e.status == LES_E_NOMEM, e.status
+else:
+    raise AssertionError("created without its memory")
+assert fake.fake_held() == 0
+""", LES_FUSE=fuse)
