@@ -955,6 +955,7 @@ void les::rows_h2d(les_ctx* c, double* d, const double* h, int ld, long rows) {
         les_note(c, hipMemcpyAsync(d, h, nx * 8 * (size_t)rows, hipMemcpyHostToDevice, c->stream));
         return;
     }
+    les_note(c, hipGetLastError());   // of earlier launches: the two below drop errors of their own
     if (!pageable(h) || !bounce_ready(c)) {
         les_note(c, hipMemcpy2DAsync(d, nx * 8, h, (size_t)ld * 8, nx * 8, (size_t)rows, hipMemcpyHostToDevice,
                                      c->stream));
@@ -982,6 +983,7 @@ void les::rows_d2h(les_ctx* c, double* h, const double* d, int ld, long rows) {
         les_note(c, hipMemcpyAsync(h, d, nx * 8 * (size_t)rows, hipMemcpyDeviceToHost, c->stream));
         return;
     }
+    les_note(c, hipGetLastError());   // of earlier launches: the two below drop errors of their own
     if (!pageable(h) || !bounce_ready(c)) {
         les_note(c, hipMemcpy2DAsync(h, (size_t)ld * 8, d, nx * 8, nx * 8, (size_t)rows, hipMemcpyDeviceToHost,
                                      c->stream));

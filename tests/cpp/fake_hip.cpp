@@ -22,7 +22,7 @@ std::map<void*, size_t> blocks;
 size_t held = 0, budget = (size_t)-1;
 long nmalloc = 0, nstream = 0;
 std::string failing;
-bool query_fails = false;
+bool query_fails = false, host_fails = false;
 hipError_t last = hipSuccess;
 hipError_t give(hipError_t e) {
     if (e != hipSuccess) last = e;
@@ -42,6 +42,7 @@ long fake_held() { return (long)held; }
 void fake_budget(long b) { budget = b < 0 ? (size_t)-1 : (size_t)b; }
 void fake_fail_kernel(const char* part) { failing = part; }
 void fake_fail_query(int on) { query_fails = on != 0; }
+void fake_fail_host_malloc(int on) { host_fails = on != 0; }
 void fake_clear() { launches.clear(); }
 long fake_nlaunch() { return (long)launches.size(); }
 const char* fake_kernel(long i) { return launches[i].kernel.c_str(); }
@@ -88,6 +89,7 @@ hipError_t hipFree(void* p) {
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    if (host_fails) return give(hipErrorOutOfMemory);
     *p = calloc(1, n);
     return hipSuccess;
 }

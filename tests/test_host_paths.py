@@ -74,3 +74,23 @@ else:
     raise AssertionError("created without its memory")
 assert fake.fake_held() == 0
 """, LES_FUSE=fuse)
+
+
+@pytest.mark.parametrize("why", ["query", "host_malloc"])
+def test_a_failed_launch_is_reported(why, fake):
+    """A launch that fails before a strided read-back is reported, also when
+    the read-back's own query of the host pointer, or its page-locked chunks,
+    fail and are done without."""
+    fake(f"""
+g = lib.create(grid(24, 12))
+ld = g.nx + 2
+out, spec, big = np.zeros((g.ny, ld)), np.zeros((g.ny, g.nx // 2 + 1, 2)), np.zeros((18, 36))
+p = lambda a: a.ctypes.data_as(C.POINTER(C.c_double))
+calls = dict(ifftn=("x_c2r", p(spec), p(out), ld), zero_unpadding=("yline", p(big), p(out), ld))
+fake.fake_fail_{why}(1)
+for name, (kernel, *args) in calls.items():
+    fake.fake_fail_kernel(kernel.encode())
+    assert g._f[name](g._h, *args) == LES_E_HIP, name
+    fake.fake_fail_kernel(b"")
+    assert g._f[name](g._h, *args) == LES_OK, name
+""")
