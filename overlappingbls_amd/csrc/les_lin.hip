@@ -46,8 +46,12 @@ namespace {
 template <typename T>
 hipError_t lalloc(les_ctx* c, T** p, size_t count) {
     void* v = nullptr;
+    les_note(c, hipGetLastError());   // of earlier launches: a refusal's own error is dropped below
     hipError_t e = hipMalloc(&v, sizeof(T) * (count ? count : 1));
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return e;
+    }
     c->allocs.push_back(v);
     *p = static_cast<T*>(v);
     return hipSuccess;

@@ -94,3 +94,26 @@ for name, (kernel, *args) in calls.items():
     fake.fake_fail_kernel(b"")
     assert g._f[name](g._h, *args) == LES_OK, name
 """)
+
+
+def test_a_refused_creation_leaves_nothing_behind(fake):
+    """After memory ran out (les_create, les_set_precision) the next calls
+    that have what they need succeed."""
+    fake("""
+g = lib.create(grid(24, 12))
+held = fake.fake_held()
+fake.fake_budget(held)
+try:
+    g.set_precision(LES_MIXED)
+except LesError as e:
+    assert e.status == LES_E_NOMEM, e.status
+else:
+    raise AssertionError("mixed mode without its memory")
+g.ddx("WORK1", "WORK0")
+try:
+    lib.create(grid(24, 12))
+except LesError as e:
+    assert e.status == LES_E_NOMEM, e.status
+fake.fake_budget(-1)
+lib.create(grid(24, 12)).close()
+""")
