@@ -765,17 +765,19 @@ void press_filter_project(les_ctx* c, int jt, bool theta_rows) {
         const Batch<double, double> fb = batch3<double, double>(u + np, v + np, w + np, u + np, v + np, w + np);
         if (!c->fuse)
             xline_real<double>(c->stream, fb, (long)(nz - 1) * c->ny, c->nx, c->nx, c->tw_x, c->tw_x, OP_NYQ, 0.0);
-        les_note(c, hipEventRecord(c->ev_xf, c->stream));
-        les_note(c, hipStreamWaitEvent(c->sums, c->ev_xf, 0));
-        yline_real<double>(c->sums, fb, nz - 1, c->nx, c->nx, c->nx, (long)np, (long)np, c->tw_y, c->tw_y, OP_NYQ,
-                           0.0);
-        les_note(c, hipEventRecord(c->ev_yf, c->sums));
+        hipStream_t ys = c->overlap ? c->sums : c->stream;
+        if (c->overlap) {
+            les_note(c, hipEventRecord(c->ev_xf, c->stream));
+            les_note(c, hipStreamWaitEvent(ys, c->ev_xf, 0));
+        }
+        yline_real<double>(ys, fb, nz - 1, c->nx, c->nx, c->nx, (long)np, (long)np, c->tw_y, c->tw_y, OP_NYQ, 0.0);
+        if (c->overlap) les_note(c, hipEventRecord(c->ev_yf, ys));
     }
     yline_spec<W>(c->stream, batch3<cx<W>, cx<W>>(Hx, Hy, Hz, Hx, Hy, Hz), nz + 1, c->lhx, (long)ns, c->tw_y, SP_FWD,
                   nullptr);
     if (modi != 0.0 && !mixed(c)) press_modi_dev(c, c->spec3[2], modi);
     press_spectra<W>(c, WF<W>(c, LES_F_P), WF<W>(c, LES_F_DPDX), WF<W>(c, LES_F_DPDY));
-    if (before) les_note(c, hipStreamWaitEvent(c->stream, c->ev_yf, 0));
+    if (before && c->overlap) les_note(c, hipStreamWaitEvent(c->stream, c->ev_yf, 0));
     gradp_project_dev<W>(c, jt, theta_rows);
     if (!before) filter3_f(c, u, v, w, (int)c->nlev);
 }
@@ -1064,7 +1066,8 @@ int les_create(const les_params* prm, les_ctx** out) {
     // same results; for checking that)
     c->fuse = 1;
     if (const char* fz = getenv("LES_FUSE")) c->fuse = strcmp(fz, "0") != 0;
-    // LES_OVERLAP=0: theta's RHS and update in order on the context's stream
+    // LES_OVERLAP=0: theta's RHS and update and the filter's y pass in order on
+    // the context's stream (the ordered plane sums keep streams of their own)
     c->overlap = 1;
     if (const char* ov = getenv("LES_OVERLAP")) c->overlap = strcmp(ov, "0") != 0;
     c->nx = prm->nxt; c->ny = prm->nyt; c->nz = prm->nzt;

@@ -134,7 +134,7 @@ struct les_ctx {
     int sgs_frozen;            // skip the Lagrangian SGS update (Cs_opt2, F_* held)
     int lin_obj;               // objective of the derivative windows (LES_OBJ_*)
     int fuse;                  // fused kernels (LES_FUSE=0 at creation: the separate ones)
-    int overlap;               // theta's RHS and update on aux (LES_OVERLAP=0: in order)
+    int overlap;               // theta's RHS and update on aux, the filter's y pass on sums (LES_OVERLAP=0: in order)
     int lag_done;              // this step's u_lag accumulation already done (k_step_begin)
     int ddz_done;              // this step's ddz of u, v, w already done (k_step_begin)
     int obk_early;             // this step's obukhov sums already launched on aux (les_run)

@@ -117,3 +117,23 @@ except LesError as e:
 fake.fake_budget(-1)
 lib.create(grid(24, 12)).close()
 """)
+
+
+@pytest.mark.parametrize("overlap", ["0", "1"])
+def test_serial_order_uses_one_stream(overlap, fake):
+    """With LES_OVERLAP=0 every kernel of a step but the ordered plane sums (and
+    the fills of their inputs) is launched on the context's stream; the filter's
+    y pass, which otherwise runs beside the pressure solve, among them."""
+    fake(f"""
+for precision in (0, LES_MIXED):
+    g = lib.create(grid(24, 12))
+    g.set_precision(precision)
+    fake.fake_clear()
+    g.run(1, 3)
+    of = launches()
+    main = [s for k, s in of if "tdma" in k][0]
+    sums = ("k_obukhov_sums", "k_level_means", "k_fill")
+    away = {{k for k, s in of if s != main and not any(n in k for n in sums)}}
+    assert bool(away) == {overlap == "1"}, away
+    g.close()
+""", LES_OVERLAP=overlap)
