@@ -4,6 +4,7 @@
 // nzt-1/nzt).  Streaming kernels are HBM-bound: one read of each input and
 // one write of each output per point, grid-stride over (level, plane).
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 #include "fft_rg.hpp"
 #include "les_lag.hpp"
@@ -212,23 +213,26 @@ __device__ __forceinline__ double wave_chain(long n, const F& val, double* lds) 
 }
 
 // The same sum by a workgroup of OS_NT threads, for planes of more than
-// OS_MIN values: the first OS_HEAD values are walked (the sum's early binades
-// are short), then chunks of OS_NT runs of OS_RUN values are scanned
+// OS_MIN values: chunks of OS_NT runs of OS_RUN values are scanned
 // (ordered_sum.hpp).  A run that may leave the sum's binade is added value by
-// value and the chunk scanned again behind it; after OS_TRIES of those (sums
-// of mixed sign about zero) the rest is walked.  Bound by latency: one
+// value and the chunk scanned again behind it; the first OS_HEAD values are
+// walked (the sum's early binades are short), and so is what is left of a
+// chunk whose scans no longer pay (SumPace).  Bound by latency: one
 // workgroup, about 2 us a scan (a third of it the runs' roundings, the rest
 // the lane scan and the two barriers).  Obukhov's sums, walk against scan,
-// alone: 28 / 15 us at 64^2, 300 / 74 us at 256^2, 810 / 262 us at 512^2; in
-// a 512 x 512 step, beside kernels that keep the memory busy, 2600 / 818 us
-// (there the wall model waited 1.2 ms for them).  At 48^2 both take 14 us:
-// smaller planes keep the walk.
-constexpr int OS_NT = 256, OS_RUN = 16, OS_HEAD = 512, OS_TRIES = 16;
+// alone: 24 / 16 us at 64^2, 345 / 77 us at 256^2, 1480 / 247 us at 512^2;
+// in a 512 x 512 step, beside kernels that keep the memory busy, 2600 / 818 us
+// (there the wall model waited 1.2 ms for them).  Plane means of v and w, which
+// take either sign, beside those of u (sponge at 256^2, 64 levels): walk 290 us,
+// u 75, v 365, w 330 us; with sixteen tries in each plane instead of SumPace's
+// rule v and w took 430 and 400 us (at 64^2: walk 21, now 30 and 22, tries 72).
+// At 48^2 both take 14 us: smaller planes keep the walk.
+constexpr int OS_NT = 256, OS_RUN = 16, OS_HEAD = 512;
 constexpr long OS_MIN = 2048;
 constexpr int OS_NW = OS_NT / 64, OS_CHUNK = OS_NT * OS_RUN;
 
 struct OsLds {
-    double x[OS_CHUNK + OS_NT];   // a chunk, one padding value per run
+    double x[OS_CHUNK + OS_NT + 2 * (OS_RUN + 1)];   // a chunk, one padding value per run; two runs read past it
     double wd[OS_NW];
     int wD[OS_NW], first[OS_NW];
     double s;
@@ -265,92 +269,111 @@ __device__ __forceinline__ SumMap wave_scan(SumMap m) {   // inclusive
     return m;
 }
 
-// s + the values i0..n-1 in order, walked by the first wavefront
-template <typename F>
-__device__ double block_walk(long i0, long n, const F& val, double s, OsLds& L) {
-    constexpr int ST = OS_CHUNK / 2, PER = ST / OS_NT;   // two stages
-    const int t = threadIdx.x;
-    int b = 0;
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const long i = i0 + j * OS_NT + t;
-        if (i < n) L.x[j * OS_NT + t] = val(i);
-    }
+// s + the values of the chunk's runs r0..r1-1 in order, walked by the first
+// wavefront
+__device__ double block_walk(int r0, int r1, double s, OsLds& L) {
     __syncthreads();
-    for (long base = i0; base < n; base += ST, b ^= 1) {
-        double v[PER];
-        const bool more = base + ST < n;
-        if (more) {
+    if (threadIdx.x < 64) {
+        // at the highest wave priority the dependent adds issue ahead of the
+        // other waves on the SIMD
+        __builtin_amdgcn_s_setprio(3);
+        // two runs at a time, the next two read while these are added (reads
+        // past the last run stay in L.x and are not added)
+        constexpr int N = 2 * OS_RUN, Q = 2 * (OS_RUN + 1);
+        const double* q = L.x + r0 * (OS_RUN + 1);
+        double a[N], b[N];
+        auto get = [&](double* w, const double* p) {
 #pragma unroll
-            for (int j = 0; j < PER; ++j) {
-                const long i = base + ST + j * OS_NT + t;
-                v[j] = val(i < n ? i : n - 1);
-            }
+            for (int e = 0; e < N; ++e) w[e] = p[e + e / OS_RUN];
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto add = [&](const double* w, int n) {
+#pragma unroll
+            for (int e = 0; e < N; ++e)
+                if (e < n) s += w[e];
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        get(a, q);
+        int runs = r1 - r0;
+        for (; runs >= 4; runs -= 4, q += 2 * Q) {
+            get(b, q + Q);
+            add(a, N);
+            get(a, q + 2 * Q);
+            add(b, N);
         }
-        if (t < 64) {
-            // at the highest wave priority the dependent adds issue ahead of
-            // the other waves on the SIMD
-            __builtin_amdgcn_s_setprio(3);
-            const int lim = (n - base < ST) ? (int)(n - base) : ST;
-            const double* q = L.x + b * ST;
-            int j = 0;
-            for (; j + 32 <= lim; j += 32) {
-                double w[32];
-#pragma unroll
-                for (int e = 0; e < 32; ++e) w[e] = q[j + e];
-                asm volatile("" ::: "memory");
-#pragma unroll
-                for (int e = 0; e < 32; ++e) s += w[e];
-            }
-            for (; j < lim; ++j) s += q[j];
-            __builtin_amdgcn_s_setprio(0);
+        if (runs >= 2) {
+            get(b, q + Q);
+            add(a, N);
+            if (runs == 3) add(b, OS_RUN);
+        } else if (runs == 1) {
+            add(a, OS_RUN);
         }
-        if (more) {
-#pragma unroll
-            for (int j = 0; j < PER; ++j) L.x[(b ^ 1) * ST + j * OS_NT + t] = v[j];
-        }
-        __syncthreads();
+        __builtin_amdgcn_s_setprio(0);
     }
-    if (t == 0) L.s = s;
+    if (threadIdx.x == 0) L.s = s;
     __syncthreads();
     return L.s;
 }
 
-template <typename F>
-__device__ double block_chain(long n, const F& val, OsLds& L) {
+// The values are cv(raw(i)): raw reads memory.
+template <typename RAW, typename CV>
+__device__ double block_chain(int n, const RAW& raw, const CV& cv, OsLds& L) {
+    using R = decltype(raw(0));
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    int tries = OS_TRIES;
-    auto load = [&](double* r, long base) {   // coalesced; s + 0 = s past the last value
+    SumPace pace;
+    double s = 0.0;
+    // coalesced; nothing but the address depends on the end of the plane, and
+    // all of a chunk's reads come before the first cv, so that no read waits
+    // for another
+    auto load = [&](double* r, int base) {
+        R q[OS_RUN];
 #pragma unroll
         for (int j = 0; j < OS_RUN; ++j) {
-            const long i = base + j * OS_NT + t;
-            const double v = val(i < n ? i : n - 1);
-            r[j] = (i < n) ? v : 0.0;
+            q[j] = raw(min(base + j * OS_NT + t, n - 1));
         }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < OS_RUN; ++j) r[j] = cv(q[j]);
     };
     // two chunks in flight: a load takes several us while other kernels keep
     // the memory busy, longer than a scan
     double n0[OS_RUN], n1[OS_RUN];
-    load(n0, OS_HEAD);
-    if (OS_HEAD + OS_CHUNK < n) load(n1, OS_HEAD + OS_CHUNK);
-    double s = block_walk(0, OS_HEAD, val, 0.0, L);
-    // adds the chunk at base, loaded in r, and refills r; true when the rest
-    // was walked
-    auto add_chunk = [&](double* r, long base) -> bool {
+    load(n0, 0);
+    if (OS_CHUNK < n) load(n1, OS_CHUNK);
+    // adds the chunk at base, loaded in r, and refills r
+    auto add_chunk = [&](double* r, int base) {
         // through LDS: thread t takes the run of values OS_RUN t ..
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < OS_RUN; ++j) {
             const int e = j * OS_NT + t;
-            L.x[e + e / OS_RUN] = r[j];
+            L.x[e + e / OS_RUN] = (base + e < n) ? r[j] : 0.0;   // s + 0 = s past the last value
         }
         __syncthreads();
-        double x[OS_RUN];
-#pragma unroll
-        for (int j = 0; j < OS_RUN; ++j) x[j] = L.x[t * (OS_RUN + 1) + j];
         if (base + 2 * OS_CHUNK < n) load(r, base + 2 * OS_CHUNK);
+        const int lim = min((n - base + OS_RUN - 1) / OS_RUN, OS_NT);   // runs of values
         int start = 0;                              // first run not yet added
-        while (start < OS_NT) {
+        bool scan = pace.chunk(base == 0);
+        if (base == 0) {
+            start = OS_HEAD / OS_RUN;
+            s = block_walk(0, start, s, L);
+            double a = 0.0;   // each wavefront forms the same sum
+#pragma unroll
+            for (int j = 0; j < OS_HEAD / 64; ++j) {
+                const int e = j * 64 + lane;
+                a += fabs(L.x[e + e / OS_RUN]);
+            }
+#pragma unroll
+            for (int o = 32; o > 0; o /= 2) a += __shfl_xor(a, o);
+            scan = !sum_cancels(s, a);
+        }
+        const bool tried = scan;
+        double x[OS_RUN];
+        if (tried) {
+#pragma unroll
+            for (int j = 0; j < OS_RUN; ++j) x[j] = L.x[t * (OS_RUN + 1) + j];
+        }
+        while (scan && start < lim) {
             const SumGrid g = sum_grid(s);
             const bool active = t >= start;
             SumMap own{0.0, 0};
@@ -379,7 +402,8 @@ __device__ double block_chain(long n, const F& val, OsLds& L) {
             for (int q = 0; q < OS_NW; ++q) stop = min(stop, L.first[q]);
             if (stop == OS_NT) {
                 s = sum_value(g, s, sum_add(all, g.odd));
-                return false;
+                start = lim;
+                break;
             }
             if (t == stop) {
                 double v = sum_value(g, s, at);
@@ -389,18 +413,19 @@ __device__ double block_chain(long n, const F& val, OsLds& L) {
             }
             __syncthreads();
             s = L.s;
+            scan = pace.stopped((stop + 1 - start) * OS_RUN);
             start = stop + 1;
-            if (--tries == 0) {
-                __syncthreads();
-                s = block_walk(base + (long)start * OS_RUN, n, val, s, L);
-                return true;
-            }
         }
-        return false;
+        if (start < lim) {
+            if (tried || base == 0) pace.gave_up();
+            s = block_walk(start, lim, s, L);
+        } else if (tried) {
+            pace.finished();
+        }
     };
-    for (long base = OS_HEAD; base < n; base += 2 * OS_CHUNK) {
-        if (add_chunk(n0, base)) break;
-        if (base + OS_CHUNK < n && add_chunk(n1, base + OS_CHUNK)) break;
+    for (int base = 0; base < n; base += 2 * OS_CHUNK) {
+        add_chunk(n0, base);
+        if (base + OS_CHUNK < n) add_chunk(n1, base + OS_CHUNK);
     }
     return s;
 }
@@ -420,7 +445,7 @@ __global__ __launch_bounds__(OS_NT) void k_level_means_scan(const double* __rest
                                                             double* __restrict__ out) {
     __shared__ OsLds L;
     const double* p = f + (long)blockIdx.x * plane;
-    const double s = block_chain(plane, [&](long i) { return p[i]; }, L);
+    const double s = block_chain((int)plane, [&](int i) { return p[i]; }, [](double v) { return v; }, L);
     if (threadIdx.x == 0) out[blockIdx.x] = s / nn;
 }
 
@@ -443,10 +468,11 @@ __device__ __forceinline__ void obukhov_sums(const SUM& sum, const double* __res
     const int which = blockIdx.x;
     double s;
     if (which == 0) {
-        s = sum([&](long i) { return sqrt(u1[i] * u1[i] + v1[i] * v1[i]); });
+        s = sum([&](int i) { return double2{u1[i], v1[i]}; },
+                [](double2 q) { return sqrt(q.x * q.x + q.y * q.y); });
     } else {
         const double* __restrict__ p = which == 1 ? psi : (which == 2 ? t3 : th1);
-        s = sum([&](long i) { return p[i]; });
+        s = sum([&](int i) { return p[i]; }, [](double v) { return v; });
     }
     if (threadIdx.x == 0) out[which] = s;
 }
@@ -456,7 +482,8 @@ __global__ __launch_bounds__(64) void k_obukhov_sums(const double* __restrict__ 
                                                       double* __restrict__ out) {
     __builtin_amdgcn_s_setprio(3);
     __shared__ __align__(16) double lds[3 * SEQ_STAGE];
-    obukhov_sums([&](const auto& val) { return wave_chain(plane, val, lds); }, u1, v1, psi, t3, th1, out);
+    obukhov_sums([&](const auto& raw, const auto& cv) { return wave_chain(plane, [&](long i) { return cv(raw((int)i)); }, lds); },
+                 u1, v1, psi, t3, th1, out);
 }
 __global__ __launch_bounds__(OS_NT) void k_obukhov_sums_scan(const double* __restrict__ u1,
                                                              const double* __restrict__ v1,
@@ -465,7 +492,8 @@ __global__ __launch_bounds__(OS_NT) void k_obukhov_sums_scan(const double* __res
                                                              const double* __restrict__ th1, long plane,
                                                              double* __restrict__ out) {
     __shared__ OsLds L;
-    obukhov_sums([&](const auto& val) { return block_chain(plane, val, L); }, u1, v1, psi, t3, th1, out);
+    obukhov_sums([&](const auto& raw, const auto& cv) { return block_chain((int)plane, raw, cv, L); }, u1, v1, psi, t3, th1,
+                 out);
 }
 static void launch_obukhov_sums(hipStream_t s, int nsums, const double* u1, const double* v1, const double* psi,
                                 const double* t3, const double* th1, long plane, double* out) {

@@ -149,4 +149,35 @@ LES_HD bool sum_inside(const SumGrid& g, double at, const SumMap& m, double mn, 
 }
 LES_HD double sum_value(const SumGrid& g, double s, double at) { return g.zero ? s : (g.S + at) * g.inv; }
 
+// When a chunk of values is scanned and when it is added one by one.  A scan
+// takes as long as walking SUM_SCAN values (3.2 us against 4.5 ns a value).
+// Sums of one sign leave a binade each time they double, and a scan reaches
+// from one such point to the next; sums of mixed sign can stay about the end
+// of a binade, where each scan advances a few values.  So the rest of a chunk
+// is walked once its scans have fallen a scan's time behind a walk, two in the
+// first chunk, where a sum of one sign stops several times; and with each such
+// chunk in a row one, two, then four chunks are walked untried.  `cancels`
+// says it of the first values at once: the sum is small beside the sum of the
+// magnitudes.
+constexpr int SUM_SCAN = 768, SUM_BACK = 4;
+struct SumPace {
+    int skip = 0, back = 1, credit = 0;
+    LES_HD bool chunk(bool first) {   // scan this chunk?
+        credit = first ? SUM_SCAN : 0;
+        if (skip == 0) return true;
+        --skip;
+        return false;
+    }
+    LES_HD bool stopped(int added) {   // a scan ended at a stop, `added` values on: scan again?
+        credit += added - SUM_SCAN;
+        return credit >= -SUM_SCAN;
+    }
+    LES_HD void gave_up() {
+        skip = back;
+        back = (back < SUM_BACK) ? 2 * back : SUM_BACK;
+    }
+    LES_HD void finished() { back = (back > 1) ? back / 2 : 1; }
+};
+LES_HD bool sum_cancels(double s, double magnitudes) { return fabs(s) * 8.0 < magnitudes; }
+
 }  // namespace les
