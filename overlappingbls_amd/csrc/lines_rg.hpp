@@ -937,11 +937,14 @@ __global__ __launch_bounds__((fused_threads<T, NIN, NOUT>())) void kr_fused_x(
 // 256 levels, 777 -> 526 us in FP64 (4.6 TB/s) and 363 -> 275 us in FP32.
 // Three levels: 559 / 287 us with two, 581 with two and the store's pointers
 // in memory, 718 / 488 with four, 666 with one.
-// NLV: as many of three levels as leave two workgroups on a CU and 512 threads,
-// with the twiddle tables in LDS (three levels with them read through the
-// vector cache: 579 / 310 us), unless that leaves one level: 768-point rows in
-// FP64 take two levels and the tables from the cache (512 x 512 x 65 levels:
-// 757 us; one level and tables in LDS 995, a block per component 937).
+// NLV: as many of three levels as leave two workgroups on a CU and 512 threads
+// (96 butterflies a 768-point row: two levels would be 576).  The twiddle
+// tables are in LDS (three levels with them read through the vector cache: 579
+// / 310 us) unless there is one level and three workgroups do not share a CU
+// with them.  768-point rows, 512 x 512 x 65 levels, FP64 / FP32, us: one level
+// with tables in LDS 978 / 370, from the cache 741 / 417; two levels in LDS
+// 768 / 404 (FP64: one workgroup a CU), from the cache 815 / 456; a block per
+// component 911 / 421.  So FP64 reads them from the cache, FP32 from LDS.
 template <typename T, int NIN, int NOUT>
 struct CrossShape {
     static constexpr int mb = cmax(rg_maxbf(NIN), rg_maxbf(NOUT));
@@ -953,11 +956,14 @@ struct CrossShape {
         while (nl > 1 && (3 * nl * mb > 512 || lds(nl, tables) > 81920)) --nl;
         return nl;
     }
-    static constexpr bool TWL = levels(true) > 1;
+    static constexpr bool TWL = levels(true) > 1 || 3 * lds(1, true) <= 163840;
     static constexpr int NLV = levels(TWL);
     static constexpr int NTH = round64(3 * NLV * mb);
     static_assert(lds(NLV, TWL) <= 81920, "two workgroups a CU");
 };
+static_assert(CrossShape<double, 384, 256>::NLV == 3 && CrossShape<double, 384, 256>::TWL, "as measured above");
+static_assert(CrossShape<double, 768, 512>::NLV == 1 && !CrossShape<double, 768, 512>::TWL, "as measured above");
+static_assert(CrossShape<float, 768, 512>::NLV == 1 && CrossShape<float, 768, 512>::TWL, "as measured above");
 template <typename T, int NIN, int NOUT>
 __global__ __launch_bounds__((CrossShape<T, NIN, NOUT>::NTH)) void kr_cross_x(
     ConvIn<T> a, T* o0, T* o1, T* o2, long nrp, int ny_in, long plane_in, const cx<T>* __restrict__ twin_g,
