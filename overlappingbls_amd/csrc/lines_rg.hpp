@@ -866,8 +866,10 @@ struct FusedWork {
 // vorticity's pads (global twiddles, so its LDS is the lines alone) take half
 // the lines of an ordinary x pass, more blocks a CU (FP64 431 -> 365 us), in
 // FP32 with twice the threads the transform has butterflies for, for the
-// loads' sake (249 -> 222 us; slower in FP64); a quarter of the lines: 698 and
-// 326 us.  The advection's unpads take the ordinary lines and twice the
+// loads' sake (249 -> 222 us; slower in FP64), unless the block is one line,
+// whose few loads a thread leave nothing to gain (384 -> 576, 29 levels: 125 us
+// with them, 93 without; 512 -> 768, 17 levels: 70 and 64 us); a quarter of the
+// lines: 698 and 326 us.  The advection's unpads take the ordinary lines and twice the
 // threads (FP64 450 -> 443, FP32 235 -> 226 us).
 template <typename T, int NIN, int NOUT>
 constexpr int fused_lines() {
@@ -876,8 +878,8 @@ constexpr int fused_lines() {
 }
 template <typename T, int NIN, int NOUT>
 constexpr int fused_threads() {
-    constexpr int mb = cmax(rg_maxbf(NIN), rg_maxbf(NOUT));
-    return round64(fused_lines<T, NIN, NOUT>() * mb) * (NIN < NOUT && sizeof(T) == 8 ? 1 : 2);
+    constexpr int mb = cmax(rg_maxbf(NIN), rg_maxbf(NOUT)), nl = fused_lines<T, NIN, NOUT>();
+    return round64(nl * mb) * (NIN < NOUT && (sizeof(T) == 8 || nl == 1) ? 1 : 2);
 }
 
 // NC components per row pair (1: the scalar advection, 3: the vorticity).
