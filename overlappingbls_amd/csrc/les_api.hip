@@ -1062,8 +1062,10 @@ int les_create(const les_params* prm, les_ctx** out) {
     if (const char* lk = getenv("LES_LINE_KERNELS")) g_use_ct = strcmp(lk, "generic") != 0;
     les_ctx* c = new les_ctx();
     c->prm = *prm;
-    // LES_FUSE=0: the separate kernels instead of the fused ones (bitwise the
-    // same results; for checking that)
+    // LES_FUSE=0: the separate kernels instead of the fused ones that have their
+    // bits, for checking that.  The pressure's row transform and the filter in
+    // front of the projection (press_filter_project) stay: the other order rounds
+    // differently, and is what statistics steps take.
     c->fuse = 1;
     if (const char* fz = getenv("LES_FUSE")) c->fuse = strcmp(fz, "0") != 0;
     // LES_OVERLAP=0: theta's RHS and update and the filter's y pass in order on

@@ -137,3 +137,25 @@ for precision in (0, LES_MIXED):
     assert bool(away) == {overlap == "1"}, away
     g.close()
 """, LES_OVERLAP=overlap)
+
+
+@pytest.mark.parametrize("fuse", ["0", "1"])
+def test_pressure_routes(fuse, fake):
+    """Plain steps form the pressure's right-hand side inside its row transform,
+    with LES_FUSE=0 too (there the filter's row pass is a kernel of its own);
+    statistics steps and rows without a table prepare it."""
+    fake(f"""
+for nx, stats in ((32, 0), (32, 1), (12, 0)):
+    g = lib.create(grid(nx, 12))
+    if stats:
+        g.set_avgslice(True, 1, 100)
+    fake.fake_clear()
+    g.run(1, 1)
+    names = [k for k, s in launches()]
+    fused = [k for k in names if "kr_x_press" in k]
+    assert bool(fused) == (nx == 32 and not stats), (nx, stats)
+    assert any("k_press_prep" in k for k in names) != bool(fused), (nx, stats)
+    if fused:
+        assert fused[0].count("Lb1") == {fuse}, fused   # the FILTER argument
+    g.close()
+""", LES_FUSE=fuse)
