@@ -2028,7 +2028,9 @@ __global__ __launch_bounds__(256) void k_max3_part(const double* __restrict__ u,
 // The passes over u, v, w that open a step in one: check_cfl's partial maxima
 // (k_max3_part, levels 1..nz-1), the vertical differences (k_ddz_uvw) and,
 // with LAG, sgs_stag's u_lag accumulation (k_lag_acc, all levels).  Twelve
-// field passes instead of fifteen; bound by HBM.
+// field passes (the separate kernels' fifteen without their own repeats), 14.3
+// by HBM counters at 256^3: part of the level neighbours is read again from
+// memory.  Bound by HBM.
 template <typename W, bool LAG>
 __global__ __launch_bounds__(256) void k_step_begin(const double* __restrict__ u, const double* __restrict__ v,
                                                     const double* __restrict__ w, W* ul, W* vl, W* wl, W* uz, W* vz,

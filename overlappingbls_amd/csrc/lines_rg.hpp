@@ -518,7 +518,7 @@ __global__ __launch_bounds__((rg_threads<T, N, N, false>())) void kr_x_r2c(Batch
 // Against a prepared right-hand side, its r2c and a filter pass behind the
 // projection this saves nine field passes of 320 in an FP64 step (with the
 // passes merged in k_step_begin and k_gradp_project: a 10-step window at 256^3
-// 105.2 ms against 109.5 ms).
+// 109.3 ms against 113.2 ms, both on one card in turn).
 // Hz's ghost levels take divtz(1) and divtz(nz) (a.lo, a.hi); Hx, Hy have
 // none.  Transformed in FP64 also for single-precision spectra (the rows are
 // FP64 state); there the level's shift is taken off the kx = 0 coefficient
